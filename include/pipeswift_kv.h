@@ -384,11 +384,14 @@ int64_t psk_paged_decode_workspace_len(int64_t num_seqs, int64_t q_len, int64_t 
  * cu_seqlens_q[b]) query tokens at rows [cu_seqlens_q[b], ...) of q and out
  * (cu_seqlens_q NULL: max_seqlen_q rows each, total_q = num_seqs *
  * max_seqlen_q); total_q is the rows of q and bounds cu_seqlens_q[num_seqs].
- * num_q_heads / num_kv_heads is at most 256.  Each workgroup reads its keys
- * once for 256 / (num_q_heads / num_kv_heads) query tokens of one kv head.
- * out rows (bf16 or f32) need 4-element alignment.  workspace: device int32,
- * at least psk_paged_prefill_workspace_len(num_seqs) words, no initial
- * contents needed.  Two launches.
+ * num_q_heads / num_kv_heads is at most 256.  A query block of 256 /
+ * (num_q_heads / num_kv_heads) tokens of one kv head reads its keys once, in one
+ * workgroup, or in several that share its keys where a step has too few blocks
+ * to fill the device.  out rows (bf16 or f32) need 4-element alignment.
+ * workspace: device int32, psk_paged_prefill_workspace_len(num_seqs) words for
+ * the current device, no initial contents needed; from 2 num_seqs + 1 words up
+ * a smaller one is taken, and the step then keeps a workgroup per block.  Two
+ * launches.
  */
 int psk_paged_prefill_attention(const void* q, int64_t q_tok_stride, int64_t q_head_stride, int q_dtype,
                                 const void* k_cache, const void* v_cache, const int64_t* k_strides,

@@ -211,13 +211,16 @@ def paged_prefill_attention(
     descales, FA's bottom-right causal rule, zero rows for missing pages, bf16
     or float32 ``out``, lse [Hq, total_q]) for any number of query tokens per
     sequence, at most ``max_seqlen_q`` each, and up to 256 query heads per kv
-    head.  One workgroup per (kv head, block of 256 / (Hq / Hkv) query tokens
-    of one sequence) streams the sequence's keys once for the whole block
-    through LDS; Q K^T runs on the bf16 MFMA over exactly converted FP8
-    values and P V on the fp16 MFMA with V exact and P rounded once to fp16
-    (at most (2^-11 + K 2^-25) max|V vd| more error for K keys), fp32 sums.
-    ``workspace``: int32 of at
-    least ``prefill_workspace_words(B)`` (allocated when absent).  The ragged
+    head.  A block of 256 / (Hq / Hkv) query tokens of one sequence and kv
+    head streams the sequence's keys once through LDS, in one workgroup or,
+    where a step has too few blocks to fill the GPU, in several that each take
+    a part of the keys and leave float32 partial results to a merge; Q K^T
+    runs on the bf16 MFMA over exactly converted FP8 values and P V on the
+    fp16 MFMA with V exact and P rounded once to fp16 (at most (2^-11 + K
+    2^-25) max|V vd| more error for K keys), fp32 sums.
+    ``workspace``: int32 of ``prefill_workspace_words(B)`` (about 68 MB, most
+    of it for the partial results; allocated when absent).  One of at least 2 B
+    + 1 words is taken too, and keeps a workgroup per block.  The ragged
     layout contract, and ``validate``, are ``paged_decode_attention``'s."""
     assert q.is_cuda and k_cache.is_cuda and v_cache.is_cuda
     assert q.dim() == 3 and q.shape[2] == HEAD_DIM and q.stride(2) == 1, "q must be [T, Hq, 128] with unit last stride"
@@ -248,9 +251,8 @@ def paged_prefill_attention(
         out = torch.empty(TQ, Hq, HEAD_DIM, dtype=torch.bfloat16, device=device)
     assert out.dtype in _OUT_CODES and out.shape == (TQ, Hq, HEAD_DIM) and out.stride(2) == 1
     lse = torch.empty(Hq, TQ, dtype=torch.float32, device=device) if return_softmax_lse else None
-    need = prefill_workspace_words(B)
-    if workspace is None or workspace.numel() < need:
-        workspace = torch.empty(max(need, 1), dtype=torch.int32, device=device)
+    if workspace is None or workspace.numel() < 2 * B + 1:
+        workspace = torch.empty(prefill_workspace_words(B), dtype=torch.int32, device=device)
     assert workspace.dtype == torch.int32 and workspace.device == device
     qd, qsb, qsh = _descale(q_descale, B, Hkv, device)
     kd, ksb, ksh = _descale(k_descale, B, Hkv, device)

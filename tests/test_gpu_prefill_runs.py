@@ -1,0 +1,118 @@
+"""GPU parity of the prefill steps that are cut into equal runs
+(``csrc/prefill_runs.hip``): few query blocks, or long cached prefixes.  The
+sizes are those where a run's bookkeeping can go wrong: one block over more
+runs than a wave has lanes, blocks that end inside and at a run, sequences
+without keys or queries, pages of sizes a wave's staged keys do and do not
+share, missing pages, and scores that outgrow a run's first maximum.  The
+oracle, bounds and helper are test_gpu_attention_prefill.py's (a run's P is
+rounded to fp16 under the same 2^15 headroom, by raising the maximum)."""
+
+import numpy as np
+import pytest
+import torch
+
+from pipeswift_amd import attention
+from tests.test_gpu_attention_prefill import _prefill_case
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("Hq,Hkv,counts,prefixes,ps,causal", [
+    (8, 1, [64], [16000], 16, True),             # two blocks of 32 tokens over 256 runs: over 64 records each
+    (8, 1, [20], [4100], 16, True),              # one partial block: waves without query rows
+    (32, 8, [100, 3, 60], [1500, 7, 2900], 16, True),
+    (32, 4, [70, 0, 33], [1200, 0, 1999], 24, True),   # an empty sequence, 24-token pages
+    (32, 4, [70, 33], [1200, 1999], 12, True),   # pages a wave's 8 keys straddle: per-thread lookups
+    (6, 2, [40, 90], [1100, 1300], 64, False),   # groups of 3, every key visible
+    (32, 8, [90, 65], [1024, 1983], 128, True),  # lengths next to stage boundaries
+    (16, 16, [300], [1724], 16, True),           # group 1: 256-token blocks
+])
+def test_runs(dev, Hq, Hkv, counts, prefixes, ps, causal):
+    lens = [c + p for c, p in zip(counts, prefixes)]
+    _prefill_case(dev, 1300 + Hq + ps + len(counts), lens, counts, Hq, Hkv, ps, causal, spare_rows=2)
+
+
+@pytest.mark.parametrize("q_dtype,out_dtype", [(torch.float8_e4m3fn, torch.bfloat16), (torch.float16, torch.float32),
+                                               (torch.float32, torch.bfloat16)])
+def test_runs_dtypes(dev, q_dtype, out_dtype):
+    _prefill_case(dev, 1400, [1800, 1200], [80, 200], 32, 4, 16, True, q_dtype=q_dtype, out_dtype=out_dtype)
+
+
+@pytest.mark.parametrize("ps", [16, 12])
+def test_runs_missing_pages(dev, ps):
+    """Missing pages read as zero rows (in the staging, also between whole stages)."""
+    _prefill_case(dev, 1410, [2300, 1100], [64, 90], 32, 8, ps, True, bad_ids=True)
+
+
+def test_runs_raise_their_maximum(dev):
+    """Scores spread over hundreds of binary orders of magnitude: weights pass
+    2^15 above the maximum of a run's first 32 keys, in every run."""
+    _prefill_case(dev, 1420, [2400, 1500], [64, 130], 32, 4, 16, True, scale=4.0)
+
+
+def test_runs_negative_score_scale(dev):
+    _prefill_case(dev, 1430, [2400], [64], 16, 2, 16, True, k_sign=-1.0)
+
+
+def test_runs_query_tokens_without_keys(dev):
+    """A sequence shorter than its queries: zeros and lse -inf, beside one that has its keys."""
+    _prefill_case(dev, 1440, [5, 3000], [20, 40], 32, 8, 16, True)
+
+
+def test_runs_in_a_graph(dev):
+    """Captured with the caller's workspace and replayed on changed lengths and
+    inputs: every replay equals the eager call, bit for bit."""
+    Hq, Hkv, ps, W = 32, 8, 16, 128
+    g = torch.Generator(device=dev).manual_seed(1450)
+    kv = torch.randn(2, W, 2, ps, Hkv, 128, generator=g, device=dev).to(torch.float8_e4m3fn)[0]
+    bt = torch.randperm(W, generator=g, device=dev).to(torch.int32).view(1, W)
+    q = torch.randn(80, Hq, 128, generator=g, device=dev).to(torch.bfloat16)
+    cu = torch.tensor([0, 80], dtype=torch.int32, device=dev)
+    lens = torch.tensor([1500], dtype=torch.int32, device=dev)
+    out = torch.empty(80, Hq, 128, dtype=torch.bfloat16, device=dev)
+    ws = torch.empty(attention.prefill_workspace_words(1), dtype=torch.int32, device=dev)
+
+    def call(o):
+        return attention.paged_prefill_attention(q, kv[:, 0], kv[:, 1], bt, lens, cu, 80, out=o, workspace=ws)
+
+    call(out)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        call(out)
+    for n in (1500, 100, 2048, 81):
+        lens.fill_(n)
+        q.normal_(generator=g)
+        out.zero_()
+        graph.replay()
+        eager = call(torch.empty_like(out))
+        torch.cuda.synchronize()
+        assert torch.equal(out.view(torch.int16), eager.view(torch.int16)), f"replay at {n} keys"
+
+
+def test_small_workspace_takes_a_workgroup_per_block(dev):
+    """A workspace of the least size taken before (2 B + 1 words) is still
+    taken: the step then runs without records, with the same results."""
+    from pipeswift_amd import _lib
+
+    Hq, Hkv, ps, n, L = 8, 2, 16, 40, 2000
+    g = torch.Generator(device=dev).manual_seed(1460)
+    W = -(-L // ps)
+    kv = torch.randn(W, 2, ps, Hkv, 128, generator=g, device=dev).to(torch.float8_e4m3fn)
+    bt = torch.arange(W, dtype=torch.int32, device=dev).view(1, W)
+    q = torch.randn(n, Hq, 128, generator=g, device=dev).to(torch.float8_e4m3fn)
+    cu = torch.tensor([0, n], dtype=torch.int32, device=dev)
+    lens = torch.tensor([L], dtype=torch.int32, device=dev)
+    want = attention.paged_prefill_attention(q, kv[:, 0], kv[:, 1], bt, lens, cu, n,
+                                             out=torch.empty(n, Hq, 128, dtype=torch.float32, device=dev))
+    got = torch.empty(n, Hq, 128, dtype=torch.float32, device=dev)
+    ws = torch.empty(3, dtype=torch.int32, device=dev)
+    k, v = kv[:, 0], kv[:, 1]
+    st = _lib.lib().psk_paged_prefill_attention(
+        q.data_ptr(), q.stride(0), q.stride(1), 3, k.data_ptr(), v.data_ptr(), _lib.i64_array(k.stride()[:3]),
+        _lib.i64_array(v.stride()[:3]), bt.data_ptr(), bt.stride(0), W, lens.data_ptr(), 1, Hq, Hkv, 128, ps, W, n, n,
+        cu.data_ptr(), 1, 128 ** -0.5, None, None, None, _lib.i64_array([0] * 6), got.data_ptr(), got.stride(0),
+        got.stride(1), 0, None, 0, ws.data_ptr(), ws.numel(), _lib.stream_handle(q.device))
+    assert st == 0, _lib.lib().psk_last_error()
+    # two kernels of the same arithmetic, P rounded to fp16 about different maxima
+    assert float((got - want).abs().max()) <= 2 * 2.0 ** -11 * float(v.float().abs().max())
