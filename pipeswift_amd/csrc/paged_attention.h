@@ -30,6 +30,11 @@ constexpr float kNegBig = -1.0e30f;  // finite "no token yet" maximum
 typedef __attribute__((address_space(1))) void gvoid;
 typedef __attribute__((address_space(3))) void lvoid;
 
+// Runs of the decode reader's balanced schedule that hold a sequence's first and last tile.
+struct RunSpan {
+  uint16_t first, last;
+};
+
 struct DecodeArgs {
   const char* q;
   int64_t q_tok_stride;   // bytes
@@ -62,8 +67,8 @@ struct DecodeArgs {
   int64_t vd_b, vd_h;
   float* part;       // partial records of G * (kHead + 2) floats: [B][Hkv][max_splits] (splits) or
                      // [(B + stream_wgs) * Hkv] (balanced schedule)
-  int32_t* prefix;   // balanced schedule: units before each sequence, [B + 1]
-  int32_t stream_wgs;  // balanced schedule: workgroups per kv head; 0 with splits
+  RunSpan* spans;    // balanced schedule: of each sequence with tokens, [B]
+  int32_t stream_wgs;  // balanced schedule: runs per kv head; 0 with splits
   int32_t seq_units;   // balanced schedule: units that stand for the start of a sequence
   char* out;
   int64_t out_tok_stride;   // bytes

@@ -36,7 +36,7 @@
 //     any other block size each lane addresses its own rows (ring_attend's GEN
 //     variant), so every block size takes the same kernels.
 //   * schedules: the balanced one (equal runs of (sequence, tile) units per
-//     workgroup across sequence boundaries, head-parallel from two sequences)
+//     workgroup across sequence boundaries, all kv heads of a token at once)
 //     by default, or an explicit split count; the waves of a workgroup merge
 //     through LDS into partial records (max, sum, accumulator per query head)
 //     in the caller's workspace, and a second kernel merges a sequence's
@@ -70,8 +70,8 @@ constexpr int kMaxRows = 16;
 constexpr float kLazy = 8.0f;        // raise the running max past 2^8 headroom only
 constexpr int kRing = 2;             // LDS tile slots per wave (ring kernel)
 constexpr int kRingPages = 1024;     // page ids of a split in the ring kernel
-// Sequences of the balanced schedule: every workgroup scans their lengths
-// (twice) and keeps the prefix in the ring's LDS.
+// Sequences of the balanced schedule: every workgroup scans their lengths and
+// keeps them and their units prefix in LDS.
 constexpr int kStreamMaxSeqs = 1024;
 static_assert(kRingPages % (kWaves * 64) == 0, "page ids are staged a whole number per thread");
 
@@ -877,17 +877,14 @@ __global__ void __launch_bounds__(kWaves * 64) decode_partial_ring_kernel(Decode
 // Balanced schedule.  Per kv head the work is a list of units: for each
 // sequence b with tokens, seq_units units that carry no work (the cost of
 // starting a sequence) and then its 16-token tiles t, ceil(len_b / 16) of
-// them; T units in all.  Run j of head h takes head h's units
-// [T j / M, T (j+1) / M), M = min(grid / Hkv, T), whatever sequences they
-// belong to: every workgroup gets the same cost in tiles and sequence starts,
-// the grid (one workgroup per resident slot) ends together,
-// and the Hkv workgroups of one j walk the same tokens of the same pages at
-// the same time (a token's kv heads share its cache rows).  Workgroup
-// j * Hkv + h runs (h, j): the heads of one run are dispatched together.  Each maximal run
-// of one sequence inside the range gives one partial record, at index
-// (b + j) * Hkv + h: the records of one (b, h) come from consecutive j, Hkv
-// apart.  Workgroup 0 also stores the units prefix (prefix[b] = units before
-// b) after the records for the combine.
+// them; T units in all.  Run j of a head takes its units [T j / M,
+// T (j + 1) / M), M = min(runs, T), whatever sequences they belong
+// to: every workgroup gets the same cost in tiles and sequence starts, and the
+// grid (one workgroup per resident slot) ends together.  Each maximal run of
+// one sequence inside the range gives one partial record, at index (b + j) *
+// Hkv + h: the records of one (b, h) come from consecutive j, Hkv apart.  The
+// runs with a sequence's first and last tile note their numbers for the
+// combine.
 __device__ __forceinline__ int tiles_of(int len) { return len > 0 ? (len + kTile - 1) / kTile : 0; }
 
 // Units of sequence b in the balanced schedule: its tiles, after a.seq_units
@@ -898,137 +895,81 @@ __device__ __forceinline__ int units_of(const DecodeArgs& a, int len) {
   return len > 0 ? tiles_of(len) + a.seq_units : 0;
 }
 
+// First unit of run j of M: floor(T j / M) for T = q M + r, from 32-bit
+// divisions (M <= 1024, so r j fits).
+__device__ __forceinline__ int64_t run_start(int T, int j, int M) {
+  const uint32_t q = uint32_t(T) / uint32_t(M), r = uint32_t(T) - q * uint32_t(M);
+  return int64_t(q) * j + (r * uint32_t(j)) / uint32_t(M);
+}
+
 // Units prefix of the batch in LDS (pref[b] = units before sequence b,
-// pref[num_seqs] = all units), by the NT threads of the workgroup; returns the
-// total.  `store` also writes it to a.prefix for the combine; `lens`, when
-// given, receives a copy of the sequence lengths.
+// pref[num_seqs] = all units) and the sequence lengths, by the NT threads of
+// the workgroup; returns the total.  The scan runs in the waves' registers with
+// two barriers: every workgroup starts with it.
 template <int NT>
-__device__ __forceinline__ int64_t scan_tiles(const DecodeArgs& a, int num_seqs, int32_t* pref, int32_t* s_scan,
-                                              bool store, int32_t* lens = nullptr) {
-  const int tid = threadIdx.x;
-  const int chunk = (num_seqs + NT - 1) / NT;
-  int sum = 0;
-  for (int i = 0; i < chunk; ++i) {
-    const int b = tid * chunk + i;
-    if (b < num_seqs) {
-      const int len = a.seq_lens[b];
-      if (lens) lens[b] = len;
-      sum += units_of(a, len);
+__device__ __forceinline__ int scan_tiles(const DecodeArgs& a, int num_seqs, int32_t* pref, int32_t* lens,
+                                          int32_t* s_wave) {
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  int carry = 0;
+  for (int c0 = 0; c0 < num_seqs; c0 += NT) {
+    const int b = c0 + tid;
+    const int len = b < num_seqs ? a.seq_lens[b] : 0;
+    const int own = units_of(a, len);
+    int x = own;  // inclusive prefix over the wave
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+      const int y = __shfl_up(x, o);
+      if (lane >= o) x += y;
     }
-  }
-  s_scan[tid] = sum;
-  __syncthreads();
-  for (int o = 1; o < NT; o <<= 1) {
-    const int v = tid >= o ? s_scan[tid - o] : 0;
+    if (c0 > 0) __syncthreads();  // the previous round's sums are read
+    if (lane == 63) s_wave[wave] = x;
     __syncthreads();
-    s_scan[tid] += v;
-    __syncthreads();
-  }
-  int run = tid > 0 ? s_scan[tid - 1] : 0;
-  for (int i = 0; i < chunk; ++i) {
-    const int b = tid * chunk + i;
-    if (b < num_seqs) {
-      pref[b] = run;
-      run += units_of(a, lens ? lens[b] : a.seq_lens[b]);
+    int before = 0, total = 0;
+#pragma unroll
+    for (int w = 0; w < NT / 64; ++w) {
+      const int t = s_wave[w];
+      before += w < wave ? t : 0;
+      total += t;
     }
+    if (b < num_seqs) {
+      pref[b] = carry + before + x - own;
+      lens[b] = len;
+    }
+    carry += total;
   }
-  if (tid == NT - 1) pref[num_seqs] = s_scan[NT - 1];
+  if (tid == 0) pref[num_seqs] = carry;
   __syncthreads();
-  if (store) {
-    for (int i = tid; i <= num_seqs; i += NT) a.prefix[i] = pref[i];
-  }
-  return pref[num_seqs];
+  return carry;
 }
 
 // The sequence b that owns unit u (the last with pref[b] <= u: sequences
 // without units share their successor's prefix) and the tile t of b that unit
-// u stands for, negative inside b's leading units.
-__device__ __forceinline__ void seek_unit(const int32_t* pref, int num_seqs, int seq_units, int64_t u, int& b,
+// u stands for, negative inside b's leading units; a 64-way search of the
+// wave (one LDS read up to 64 sequences, two up to 4096).
+__device__ __forceinline__ void seek_unit(const int32_t* pref, int num_seqs, int seq_units, int64_t u, int lane, int& b,
                                           int& t) {
-  int lo = 0, hi = num_seqs - 1;
-  while (lo < hi) {
-    const int mid = (lo + hi + 1) >> 1;
-    if (pref[mid] <= u) lo = mid; else hi = mid - 1;
+  int lo = 0, n = num_seqs;  // the answer lies in [lo, lo + n) and pref[lo] <= u
+  while (n > 1) {
+    const int step = (n + 63) / 64;
+    const uint64_t m = __ballot(lane * step < n && pref[lo + lane * step] <= u);  // a prefix of the lanes
+    const int last = 63 - __builtin_clzll(m);
+    lo += last * step;
+    n = min(step, n - last * step);
   }
-  b = lo;
+  b = __builtin_amdgcn_readfirstlane(lo);
   t = int(u - pref[b]) - seq_units;
 }
 
-// Three waves per SIMD: left to itself the compiler keeps the MFMA accumulators in
-// AGPRs, which puts the general-page variant at 141 VGPRs + 36 AGPRs and two waves
-// per SIMD; asked for three it fits every variant in 143 VGPRs without spilling.
-template <int NG, bool GEN>
-__global__ void __launch_bounds__(kWaves * 64) __attribute__((amdgpu_waves_per_eu(3)))
-decode_partial_stream_kernel(DecodeArgs a, int q_dtype, int num_seqs) {
-  const int w = blockIdx.x;
-  const int lane = threadIdx.x & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(int(threadIdx.x) >> 6);
-  const int Hkv = a.num_kv_heads;
-  __shared__ RingLds lds;
-  static_assert(sizeof(lds.ring) >= sizeof(float) * kWaves * NG * kHead, "the ring doubles as the merge buffer");
-  static_assert(sizeof(lds.ring) / sizeof(int32_t) > kStreamMaxSeqs, "the ring holds the units prefix");
-
-  // units prefix over the sequences, scanned in the ring (free until the first tile)
-  int32_t* pref = reinterpret_cast<int32_t*>(&lds.ring[0][0][0][0]);
-  __shared__ int32_t s_scan[kWaves * 64];
-  const int64_t T = scan_tiles<kWaves * 64>(a, num_seqs, pref, s_scan, w == 0);
-  // no more runs than units, so that no range is empty and the records of one
-  // (b, h) stay consecutive; the other workgroups leave
-  const int h = w % Hkv, j = w / Hkv;
-  const int64_t M = min<int64_t>(gridDim.x / Hkv, T);
-  if (j >= M) return;  // uniform over the workgroup
-  int64_t u = T * j / M;
-  const int64_t u_end = T * (j + 1) / M;
-  int b, t;
-  seek_unit(pref, num_seqs, a.seq_units, u, b, t);
-  // ring_attend's first barrier orders these prefix reads before the ring is refilled
-
-  const int piece = staging_piece(a, kTile * kWaves);
-  while (u < u_end && b < num_seqs) {
-    if (t < 0) {  // leading units of b: no work
-      const int skip = int(min<int64_t>(-t, u_end - u));
-      u += skip;
-      t += skip;
-      if (u >= u_end) break;
-    }
-    const int len = a.seq_lens[b];
-    const int tb = tiles_of(len);
-    const int n = int(min<int64_t>(tb - t, u_end - u));
-    bf16x8 qop[4];
-    float sl = 0.0f;
-    BalancedState<NG> st;
-    softmax_init(st);
-    const int t_end = min(len, (t + n) * kTile);
-    for (int t0 = t * kTile; t0 < t_end; t0 += piece) {
-      const bool head = t0 == t * kTile;
-      ring_attend<NG, kWaves, kWaves, kRing, GEN>(a, st, qop, sl, b, h, t0, min(t_end, t0 + piece), len, lane, wave,
-                                                  wave, lds, [&] {
-        if (head) sl = load_head<NG, !kPvMfma && (NG <= 4)>(a, q_dtype, b, h, lane, qop);
-      });
-    }
-    __syncthreads();  // every wave is done with the ring: it becomes the merge buffer
-    write_partial<NG>(a, st, (int64_t(b) + j) * Hkv + h, lane, wave,
-                      reinterpret_cast<float(*)[NG][kHead]>(&lds.ring[0][0][0][0]));
-    u += n;
-    t += n;
-    if (t == tb) {
-      t = -a.seq_units;
-      do ++b; while (b < num_seqs && a.seq_lens[b] <= 0);
-    }
-  }
-}
-
-// Head-parallel balanced schedule.  The same units and runs as
-// decode_partial_stream_kernel, but one workgroup of kHeadWaves waves takes a
-// run for HG kv heads at once: wave w serves head hg * HG + w % HG and tile
-// phase w / HG (P = kHeadWaves / HG phases).  With HG = 8 every wave walks
+// One workgroup of kHeadWaves waves takes a run for HG kv heads at once: wave
+// w serves head hg * HG + w % HG and tile phase w / HG (P = kHeadWaves / HG
+// phases).  With HG = 8 every wave walks
 // all of the run's tiles for its own head, so at any moment one CU requests
 // whole 1 KiB token rows (all heads' 128-byte slices of a token) instead of
 // each of eight workgroups on eight XCDs requesting its own slice: a
 // read-only probe of config 2's pages streams 6.9 TB/s that way against 5.9
 // for head slices.  Workgroup j * NHG + hg serves run j of head group hg
-// (NHG = Hkv / HG); records and the units prefix are laid out as in the
-// per-head balanced schedule, so the same combine reads them.
+// (NHG = Hkv / HG).  One long sequence takes it too: 131072 tokens of 8 kv
+// heads 53.7 us against 58.3 with a 4-wave workgroup per head and run.
 constexpr int kHeadWaves = 8;
 // LDS tile slots per wave.  At one workgroup per CU deeper rings cost no
 // occupancy, but measured slower on config 2: 227 us at three against 225.
@@ -1162,16 +1103,18 @@ __global__ void __launch_bounds__(kHeadWaves * 64) decode_partial_heads_kernel(D
 
   // units prefix and lengths of the sequences, kept in LDS for the whole run
   __shared__ int32_t s_pref[kStreamMaxSeqs + 1], s_len[kStreamMaxSeqs];
-  __shared__ int32_t s_scan[W * 64];
-  const int64_t T = scan_tiles<W * 64>(a, num_seqs, s_pref, s_scan, w == 0, s_len);
+  __shared__ int32_t s_scan[W];
+  const int T = scan_tiles<W * 64>(a, num_seqs, s_pref, s_len, s_scan);
   const int hg = w % NHG, j = w / NHG;
   const int h = hg * HG + wave % HG, phase = wave / HG;
-  const int64_t M = min<int64_t>(gridDim.x / NHG, T);
+  // no more runs than units, so that no run is empty and the records of one
+  // (b, h) stay consecutive; the other workgroups leave
+  const int M = min(int(gridDim.x) / NHG, T);
   if (j >= M) return;  // uniform over the workgroup
-  int64_t u = T * j / M;
-  const int64_t u_end = T * (j + 1) / M;
+  int64_t u = run_start(T, j, M);
+  const int64_t u_end = run_start(T, j + 1, M);
   int b, t;
-  seek_unit(s_pref, num_seqs, a.seq_units, u, b, t);
+  seek_unit(s_pref, num_seqs, a.seq_units, u, lane, b, t);
 
   // page-id staging pieces: whole multiples of every phase stride
   const int piece = staging_piece(a, kTile * W);
@@ -1185,6 +1128,10 @@ __global__ void __launch_bounds__(kHeadWaves * 64) decode_partial_heads_kernel(D
     const int len = s_len[b];
     const int tb = tiles_of(len);
     const int n = int(min<int64_t>(tb - t, u_end - u));
+    if (hg == 0 && threadIdx.x == 0) {
+      if (t == 0) a.spans[b].first = uint16_t(j);
+      if (t + n == tb) a.spans[b].last = uint16_t(j);
+    }
     bf16x8 qop[4];
     float sl = 0.0f;
     BalancedState<NG> st;
@@ -1293,18 +1240,12 @@ __global__ void __launch_bounds__(64 * kCombineMaxWaves) decode_combine_kernel(D
   int64_t rs = rec;   // floats between consecutive records of (b, h)
   int n = 0;          // records of (b, h): the same for every kv head of b
   if (a.stream_wgs > 0) {
-    // run j of head h took units [T j / M, T (j+1) / M); unit u belongs to run
-    // j(u) = ((u + 1) M - 1) / T, and b owns units [p0, p0 + units), of which
-    // the first seq_units carry no work: the runs of its tiles wrote records
-    const int64_t p0 = a.prefix[b], units = a.prefix[b + 1] - p0;
-    if (units > 0) {
-      const int64_t T = a.prefix[gridDim.y];
-      const int64_t M = min<int64_t>(a.stream_wgs, T);  // as the partial kernel caps it
-      const int64_t u0 = p0 + a.seq_units, u1 = p0 + units - 1;  // first and last tile units
-      const int64_t j0 = ((u0 + 1) * M - 1) / T, j1 = ((u1 + 1) * M - 1) / T;
-      first = (int64_t(b) + j0) * a.num_kv_heads + h;
+    // the runs with b's first and last tile, and those between, left records
+    const RunSpan span = a.spans[b];
+    if (a.seq_lens[b] > 0) {
+      first = (int64_t(b) + span.first) * a.num_kv_heads + h;
       rs = int64_t(a.num_kv_heads) * rec;
-      n = int(j1 - j0 + 1);
+      n = span.last - span.first + 1;
     }
   } else {
     const int len = a.seq_lens[b];
@@ -1318,6 +1259,18 @@ __global__ void __launch_bounds__(64 * kCombineMaxWaves) decode_combine_kernel(D
   float o[CPL];
 #pragma unroll
   for (int k = 0; k < CPL; ++k) o[k] = 0.0f;
+  // 8-byte loads: records are G (kHead + 2) floats apart and their columns
+  // start 2 G floats in, so only 8-byte alignment holds for every G
+  auto load_columns = [&](int c0, int s0, int cnt, f32x2 (&x)[NB][CPL / 2]) {
+#pragma unroll
+    for (int i = 0; i < NB; ++i) {
+      // past cnt (or on a dead row) re-read a loaded record; its weight is 0
+      const int r = live ? c0 + min(s0 + i, cnt - 1) : 0;
+      const f32x2* src = reinterpret_cast<const f32x2*>(live ? col + int64_t(r) * rs : a.part);
+#pragma unroll
+      for (int k = 0; k < CPL / 2; ++k) x[i][k] = src[k];
+    }
+  };
   const int r_end = int(int64_t(n) * (w + 1) / S);
   for (int c0 = int(int64_t(n) * w / S); c0 < r_end; c0 += L) {  // uniform over the wave
     const int cnt = min(L, r_end - c0);
@@ -1326,6 +1279,8 @@ __global__ void __launch_bounds__(64 * kCombineMaxWaves) decode_combine_kernel(D
       m = part[int64_t(c0 + c) * rs + g];
       l = part[int64_t(c0 + c) * rs + G + g];
     }
+    f32x2 x[NB][CPL / 2];
+    load_columns(c0, 0, cnt, x);  // the first records' columns, in flight with their maxima and sums
     const float cm = __builtin_fmaxf(mx, group_max<L>(m));
     const float sc = __builtin_amdgcn_exp2f(mx - cm);
     den *= sc;
@@ -1335,17 +1290,7 @@ __global__ void __launch_bounds__(64 * kCombineMaxWaves) decode_combine_kernel(D
     const float wl = __builtin_amdgcn_exp2f(m - cm);  // 0 past cnt and on dead rows
     den += group_sum<L>(l * wl);
     for (int s0 = 0; s0 < cnt; s0 += NB) {
-      // 8-byte loads: records are G (kHead + 2) floats apart and their columns
-      // start 2 G floats in, so only 8-byte alignment holds for every G
-      f32x2 x[NB][CPL / 2];
-#pragma unroll
-      for (int i = 0; i < NB; ++i) {
-        // past cnt (or on a dead row) re-read a loaded record; its weight is 0
-        const int r = live ? c0 + min(s0 + i, cnt - 1) : 0;
-        const f32x2* src = reinterpret_cast<const f32x2*>(live ? col + int64_t(r) * rs : a.part);
-#pragma unroll
-        for (int k = 0; k < CPL / 2; ++k) x[i][k] = src[k];
-      }
+      if (s0 > 0) load_columns(c0, s0, cnt, x);
 #pragma unroll
       for (int i = 0; i < NB; ++i) {
         // record s0 + i's weight from lane s0 + i of the row (uniform: readlane)
@@ -1421,41 +1366,6 @@ int decode_split(int64_t max_seq_len, int64_t num_splits, int64_t seq_heads) {
   return int(std::min<int64_t>(split, INT32_MAX / 2));
 }
 
-// Workgroups of the balanced schedule on the current device: one per slot that
-// can be resident at once (CUs x occupancy of the kernel instantiation).  The
-// general-page variants launch the same grid, so that the workspace size does
-// not depend on the block size.
-template <int NG>
-int64_t stream_wgs_for() {
-  static std::mutex mu;
-  static std::map<int, int64_t> cache;
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess) return 0;
-  std::lock_guard<std::mutex> lock(mu);
-  auto it = cache.find(dev);
-  if (it != cache.end()) return it->second;
-  int cus = 0, per_cu = 0;
-  if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
-      hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, decode_partial_stream_kernel<NG, false>, kWaves * 64, 0) !=
-          hipSuccess)
-    return 0;
-  const int64_t n = int64_t(cus) * std::max(per_cu, 1);
-  cache[dev] = n;
-  return n;
-}
-
-int64_t stream_wgs(int ng) {
-  switch (ng) {
-    case 1: return stream_wgs_for<1>();
-    case 2: return stream_wgs_for<2>();
-    case 4: return stream_wgs_for<4>();
-    case 8: return stream_wgs_for<8>();
-    default:
-      if constexpr (kPvMfma) return stream_wgs_for<16>();
-      return 0;
-  }
-}
-
 int group_ng(int64_t G) { return G == 1 ? 1 : G == 2 ? 2 : G <= 4 ? 4 : G <= 8 ? 8 : 16; }
 
 // kv heads per workgroup of the head-parallel schedule: the largest of 8, 4,
@@ -1505,7 +1415,7 @@ int64_t heads_runs(int ng, int64_t num_kv_heads) {
       if constexpr (kPvMfma) slots = heads_wgs_ng<16>(hg);
       break;
   }
-  return slots > 0 ? std::max<int64_t>(1, slots / (num_kv_heads / hg)) : 0;
+  return slots > 0 ? std::min<int64_t>(1024, std::max<int64_t>(1, slots / (num_kv_heads / hg))) : 0;
 }
 
 template <int NG, bool GEN>
@@ -1519,14 +1429,13 @@ void launch_heads_ng(const DecodeArgs& a, int q_dtype, int hg, dim3 grid, hipStr
   }
 }
 
-// The partial kernels of one schedule for group slot ng: the balanced
-// schedule's head-parallel (heads) or per-head kernel with `runs` > 0, else
-// one workgroup per (split, kv head, sequence).
+// The partial kernels for group slot ng: the balanced schedule with `runs` >
+// 0, else one workgroup per (split, kv head, sequence).
 template <bool GEN>
-void launch_partials(const DecodeArgs& a, int q_dtype, int ng, int64_t runs, bool heads, int64_t num_kv_heads,
+void launch_partials(const DecodeArgs& a, int q_dtype, int ng, int64_t runs, int64_t num_kv_heads,
                      dim3 grid, hipStream_t st, int ns) {
   const dim3 block(kWaves * 64);
-  if (runs > 0 && heads) {
+  if (runs > 0) {
     const int hg = heads_hg(num_kv_heads);
     const dim3 sgrid{unsigned(runs * (num_kv_heads / hg)), 1u, 1u};
     switch (ng) {
@@ -1536,18 +1445,6 @@ void launch_partials(const DecodeArgs& a, int q_dtype, int ng, int64_t runs, boo
       case 8: launch_heads_ng<8, GEN>(a, q_dtype, hg, sgrid, st, ns); break;
       default:
         if constexpr (kPvMfma) launch_heads_ng<16, GEN>(a, q_dtype, hg, sgrid, st, ns);
-        break;
-    }
-  } else if (runs > 0) {
-    const dim3 sgrid{unsigned(runs * num_kv_heads), 1u, 1u};
-    switch (ng) {
-      case 1: hipLaunchKernelGGL((decode_partial_stream_kernel<1, GEN>), sgrid, block, 0, st, a, q_dtype, ns); break;
-      case 2: hipLaunchKernelGGL((decode_partial_stream_kernel<2, GEN>), sgrid, block, 0, st, a, q_dtype, ns); break;
-      case 4: hipLaunchKernelGGL((decode_partial_stream_kernel<4, GEN>), sgrid, block, 0, st, a, q_dtype, ns); break;
-      case 8: hipLaunchKernelGGL((decode_partial_stream_kernel<8, GEN>), sgrid, block, 0, st, a, q_dtype, ns); break;
-      default:
-        if constexpr (kPvMfma)
-          hipLaunchKernelGGL((decode_partial_stream_kernel<16, GEN>), sgrid, block, 0, st, a, q_dtype, ns);
         break;
     }
   } else {
@@ -1563,36 +1460,9 @@ void launch_partials(const DecodeArgs& a, int q_dtype, int ng, int64_t runs, boo
   }
 }
 
-// Workgroups per kv head of the balanced schedule.
-int64_t stream_runs(int ng, int64_t num_kv_heads) {
-  const int64_t slots = stream_wgs(ng);
-  return slots > 0 ? std::max<int64_t>(1, slots / num_kv_heads) : 0;
-}
-
-// The head-parallel schedule from kHeadsMinSeqs sequences up; a single
-// sequence takes the per-head schedule, whose 4-wave workgroups put more waves
-// on it.  Measured with P V on the matrix cores: from 2 sequences the
-// head-parallel schedule is faster (2 x 32768 tokens 32.8 us against 35.1,
-// 4 x 16384 32.5 against 34.8, 7 mixed 27.5 against 30.8, 3 skewed 45.5
-// against 52.4; 6 x 2048 at group 8 20.9 against 19.3), config 2's 128
-// sequences 223 us against 266 before it.
-constexpr int64_t kHeadsMinSeqs = 2;
-
 // Units that stand for the fixed cost of starting a sequence in a run (see
-// units_of), per schedule.
-#ifndef PSK_HEADS_SEQ_UNITS
-#define PSK_HEADS_SEQ_UNITS 8
-#endif
-#ifndef PSK_STREAM_SEQ_UNITS
-#define PSK_STREAM_SEQ_UNITS 0
-#endif
-constexpr int kHeadsSeqUnits = PSK_HEADS_SEQ_UNITS;
-constexpr int kStreamSeqUnits = PSK_STREAM_SEQ_UNITS;
-
-// Runs per workgroup family of the balanced schedule for this batch.
-int64_t balanced_runs(int ng, int64_t num_seqs, int64_t num_kv_heads) {
-  return num_seqs >= kHeadsMinSeqs ? heads_runs(ng, num_kv_heads) : stream_runs(ng, num_kv_heads);
-}
+// units_of).
+constexpr int kSeqUnits = 8;
 
 }  // namespace
 
@@ -1609,9 +1479,9 @@ int64_t psk_paged_decode_workspace_len(int64_t num_seqs, int64_t q_len, int64_t 
       std::max<int64_t>(1, ceil_div(max_seq_len, decode_split(max_seq_len, num_splits, num_seqs * num_kv_heads)));
   int64_t need = num_seqs * num_kv_heads * splits * rec;
   if (num_splits == 0 && num_seqs <= kStreamMaxSeqs && G <= kMaxRows) {
-    // the balanced schedule: a record per (sequence, kv head) and per workgroup, then the units prefix
+    // the balanced schedule: a record per (sequence, kv head) and per (run, kv head), then the spans
     need = std::max(need,
-                    (num_seqs + balanced_runs(group_ng(G), num_seqs, num_kv_heads)) * num_kv_heads * rec + num_seqs + 1);
+                    (num_seqs + heads_runs(group_ng(G), num_kv_heads)) * num_kv_heads * rec + num_seqs + 1);
   }
   return need;
 }
@@ -1718,15 +1588,14 @@ int psk_paged_decode_attention(const void* q, int64_t q_tok_stride, int64_t q_he
   // 16 (and its rows are within 32-bit offsets): wave-uniform tile addressing;
   // any other block size takes the general-page variants
   const bool uniform = a.bs_shift >= 4 && 16 * std::max(a.k_row, a.v_row) < (int64_t(1) << 31);
-  const bool heads = num_seqs >= kHeadsMinSeqs;
-  const int64_t runs = num_splits == 0 && num_seqs <= kStreamMaxSeqs ? balanced_runs(ng, num_seqs, num_kv_heads) : 0;
+  const int64_t runs = num_splits == 0 && num_seqs <= kStreamMaxSeqs ? heads_runs(ng, num_kv_heads) : 0;
   if (runs > 0) {
     a.stream_wgs = int32_t(runs);
-    a.seq_units = heads ? kHeadsSeqUnits : kStreamSeqUnits;
-    a.prefix = reinterpret_cast<int32_t*>(workspace + (num_seqs + runs) * num_kv_heads * G * (kHead + 2));
+    a.seq_units = kSeqUnits;
+    a.spans = reinterpret_cast<RunSpan*>(workspace + (num_seqs + runs) * num_kv_heads * G * (kHead + 2));
   }
-  if (uniform) launch_partials<false>(a, q_dtype, ng, runs, heads, num_kv_heads, grid, st, int(num_seqs));
-  else launch_partials<true>(a, q_dtype, ng, runs, heads, num_kv_heads, grid, st, int(num_seqs));
+  if (uniform) launch_partials<false>(a, q_dtype, ng, runs, num_kv_heads, grid, st, int(num_seqs));
+  else launch_partials<true>(a, q_dtype, ng, runs, num_kv_heads, grid, st, int(num_seqs));
   const int st1 = check_launch("decode partial kernel launch");
   if (st1 != PSK_OK) return st1;
   // waves per workgroup in the combine: one per combine_batch() records a
