@@ -618,58 +618,8 @@ __global__ void __launch_bounds__(256) paged_gather_kernel(GatherGeom g) {
     qs.neg = 0u;
   }
 
-  // Sequence lookup without a chain of dependent loads.  The lanes hold a
-  // window of 64 sequences k = wbase + lane: cu[k], cu[k+1] and seq_starts[k]
-  // (clamped loads, lanes past the batch hold an end of INT32_MAX).  Token t
-  // belongs to sequence wbase + n, n = the number of window entries with
-  // cu[k+1] <= t (a ballot); its cu[b] and start come from lane n.  The first
-  // window is loaded unconditionally; a batch of more than 64 sequences whose
-  // token lies beyond it places the window with one 64-wide probe of cu[64j].
-  // A later token of the chunk past the window takes the scalar walk.
-  const int32_t* sp = g.starts ? g.starts : g.cu;
-  const int64_t last = g.batch > 0 ? g.batch - 1 : 0;
-  int64_t wbase = 0;
-  int64_t kw = lane;
-  int64_t cu_lo = g.cu[kw < g.batch ? kw : g.batch];
-  int64_t cu_hi = g.cu[kw < g.batch ? kw + 1 : g.batch];
-  int32_t st = sp[kw < last ? kw : last];
-  if (g.batch > kWave && t0 >= int64_t(__builtin_amdgcn_readlane(int(cu_hi), kWave - 1))) {
-    const int64_t k = (int64_t(lane) + 1) * kWave;
-    const int64_t c = g.cu[k <= g.batch ? k : g.batch];
-    wbase = int64_t(__popcll(__ballot(k <= g.batch && c <= t0))) * kWave;
-    kw = wbase + lane;
-    cu_lo = g.cu[kw < g.batch ? kw : g.batch];
-    cu_hi = g.cu[kw < g.batch ? kw + 1 : g.batch];
-    st = sp[kw < last ? kw : last];
-  }
-  if (kw >= g.batch) cu_hi = INT32_MAX;
-  if (!g.starts) st = 0;
-  const int64_t cu0 = g.cu[0];
-
-  int64_t bseq[CH], pos[CH];
-  int nwin[CH];
-  bool slow = false;
-#pragma unroll
-  for (int c = 0; c < CH; ++c) {
-    const int64_t t = t0 + c;
-    const int n = __popcll(__ballot(cu_hi <= t));
-    nwin[c] = n;
-    slow |= n == kWave;
-    const int nl = n < kWave ? n : kWave - 1;
-    bseq[c] = wbase + n;
-    pos[c] = int64_t(__builtin_amdgcn_readlane(st, nl)) + t - int64_t(__builtin_amdgcn_readlane(int(cu_lo), nl));
-  }
-  if (slow) {  // a token of this chunk lies past the window: walk on from its end
-#pragma unroll
-    for (int c = 0; c < CH; ++c) {
-      if (nwin[c] != kWave) continue;
-      const int64_t t = t0 + c;
-      int64_t b = wbase + kWave;
-      while (b < g.batch && t >= int64_t(g.cu[b + 1])) ++b;
-      bseq[c] = b;
-      pos[c] = b < g.batch ? (g.starts ? int64_t(g.starts[b]) : 0) + t - int64_t(g.cu[b]) : 0;
-    }
-  }
+  int64_t bseq[CH], pos[CH], cu0;
+  find_rows<CH>(g.cu, g.starts, g.batch, t0, lane, bseq, pos, cu0);
 
   // Block-table reads through an always-valid pointer, the value passed
   // through readfirstlane before the select: a select between a loaded value

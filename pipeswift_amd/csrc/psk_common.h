@@ -142,6 +142,66 @@ template <> struct BufIO<1> {
   __device__ static void store(uint8_t v, __amdgpu_buffer_rsrc_t r, uint32_t off) { __builtin_amdgcn_raw_buffer_store_b8(v, r, off, 0, 2); }
 };
 
+// The sequence bseq[c] of token t0 + c of a gather and its position pos[c] in
+// it (seq_starts included), for the CH tokens of a wave; bseq[c] >= batch past
+// the last sequence.
+//
+// Sequence lookup without a chain of dependent loads.  The lanes hold a
+// window of 64 sequences k = wbase + lane: cu[k], cu[k+1] and seq_starts[k]
+// (clamped loads, lanes past the batch hold an end of INT32_MAX).  Token t
+// belongs to sequence wbase + n, n = the number of window entries with
+// cu[k+1] <= t (a ballot); its cu[b] and start come from lane n.  The first
+// window is loaded unconditionally; a batch of more than 64 sequences whose
+// token lies beyond it places the window with one 64-wide probe of cu[64j].
+// A later token of the chunk past the window takes the scalar walk.
+template <int CH>
+__device__ __forceinline__ void find_rows(const int32_t* cu, const int32_t* starts, int64_t batch, int64_t t0, int lane,
+                                          int64_t (&bseq)[CH], int64_t (&pos)[CH], int64_t& cu0) {
+  const int32_t* sp = starts ? starts : cu;
+  const int64_t last = batch > 0 ? batch - 1 : 0;
+  int64_t wbase = 0;
+  int64_t kw = lane;
+  int64_t cu_lo = cu[kw < batch ? kw : batch];
+  int64_t cu_hi = cu[kw < batch ? kw + 1 : batch];
+  int32_t st = sp[kw < last ? kw : last];
+  if (batch > kWave && t0 >= int64_t(__builtin_amdgcn_readlane(int(cu_hi), kWave - 1))) {
+    const int64_t k = (int64_t(lane) + 1) * kWave;
+    const int64_t c = cu[k <= batch ? k : batch];
+    wbase = int64_t(__popcll(__ballot(k <= batch && c <= t0))) * kWave;
+    kw = wbase + lane;
+    cu_lo = cu[kw < batch ? kw : batch];
+    cu_hi = cu[kw < batch ? kw + 1 : batch];
+    st = sp[kw < last ? kw : last];
+  }
+  if (kw >= batch) cu_hi = INT32_MAX;
+  if (!starts) st = 0;
+  cu0 = cu[0];
+
+  int nwin[CH];
+  bool slow = false;
+#pragma unroll
+  for (int c = 0; c < CH; ++c) {
+    const int64_t t = t0 + c;
+    const int n = __popcll(__ballot(cu_hi <= t));
+    nwin[c] = n;
+    slow |= n == kWave;
+    const int nl = n < kWave ? n : kWave - 1;
+    bseq[c] = wbase + n;
+    pos[c] = int64_t(__builtin_amdgcn_readlane(st, nl)) + t - int64_t(__builtin_amdgcn_readlane(int(cu_lo), nl));
+  }
+  if (slow) {  // a token of this chunk lies past the window: walk on from its end
+#pragma unroll
+    for (int c = 0; c < CH; ++c) {
+      if (nwin[c] != kWave) continue;
+      const int64_t t = t0 + c;
+      int64_t b = wbase + kWave;
+      while (b < batch && t >= int64_t(cu[b + 1])) ++b;
+      bseq[c] = b;
+      pos[c] = b < batch ? (starts ? int64_t(starts[b]) : 0) + t - int64_t(cu[b]) : 0;
+    }
+  }
+}
+
 template <int DT> struct Elt;
 template <> struct Elt<PSK_DTYPE_F32> {
   using Bits = uint32_t;
