@@ -449,6 +449,95 @@ bool launch_packed_rows(const ScatterGeom& g, const ScatterPart& p0, const Scatt
   return true;
 }
 
+// Prefill-sized quantizing appends of flat rows of a power of two of vectors.
+// A wave takes 128 vectors in a row of one part's flat (token, vector) space:
+// lane l loads vectors l and 64 + l (whole lines per load), and after the
+// conversion neighbouring lanes exchange halves, so that an even lane stores
+// vectors l, l + 1 and an odd one 64 + l - 1, 64 + l as one 16-byte store: half
+// the write requests of a store per vector, and no idle lanes on rows shorter
+// than 64 vectors.  WIDE: rows of at least 128 vectors, whose token and slot
+// are the wave's (scalar loads); otherwise they are the lane's.  A wave per
+// (token, part) against this, bf16 to FP8 in us, K and V of 128 elements:
+//   tokens       1024           4096           16384            32768
+//   1 head    2.45 / 2.37    3.77 / 2.66     8.97 /  3.74    15.76 /  6.10
+//   2 heads   2.44 / 2.41    3.91 / 3.08     9.49 /  6.08    16.57 / 10.59
+//   4 heads   2.54 / 2.57    4.47 / 3.68    10.81 / 10.84    19.39 / 19.97
+//   8 heads   3.69 / 3.13    6.66 / 6.13    20.02 / 20.21    37.80 / 38.16
+template <class C, bool WIDE>
+__global__ void __launch_bounds__(256) quant_pair_scatter_kernel(ScatterGeom g, ScatterPart p0, ScatterPart p1,
+                                                                 int row_shift) {
+  static_assert(C::IN_B == 16 && C::OUT_B == 8, "eight 16-bit elements a vector");
+  const int lane = threadIdx.x & (kWave - 1);
+  const int64_t wave = int64_t(blockIdx.x) * 4 + __builtin_amdgcn_readfirstlane(int(threadIdx.x) / kWave);
+  const int part = int(wave & 1);
+  const int64_t f0 = (wave >> 1) * (2 * kWave);  // the wave's first vector
+  const char* src = part ? p1.src : p0.src;
+  char* dst = part ? p1.dst : p0.dst;
+  const float* scale_p = part ? p1.scale : p0.scale;
+  const int64_t src_stride = part ? p1.src_stride : p0.src_stride;
+  const int64_t blk_stride = part ? p1.blk_stride : p0.blk_stride;
+  const int64_t page_stride = part ? p1.page_stride : p0.page_stride;
+  const int64_t dst_off = part ? p1.dst_off : p0.dst_off;
+  const int64_t mask = (int64_t(1) << row_shift) - 1;
+  const int odd = lane & 1;
+  typename C::In va{}, vb{};
+  int64_t slot, io;  // the slot of the pair this lane stores, and the pair's first vector in its row
+  if constexpr (WIDE) {
+    const int64_t t = f0 >> row_shift;
+    if (t >= g.num_tokens) return;
+    const int64_t i0 = f0 & mask;
+    const char* row = src + t * src_stride + i0 * C::IN_B;
+    va = vload_nt<C::IN_B>(row + lane * C::IN_B);
+    vb = vload_nt<C::IN_B>(row + (kWave + lane) * C::IN_B);
+    slot = g.slots[t];
+    io = i0 + (odd ? kWave + lane - 1 : lane);
+  } else {
+    const int64_t fa = f0 + lane, fb = fa + kWave;
+    const int64_t ta = fa >> row_shift, tb = fb >> row_shift;
+    if (ta < g.num_tokens) va = vload_nt<C::IN_B>(src + ta * src_stride + (fa & mask) * C::IN_B);
+    if (tb < g.num_tokens) vb = vload_nt<C::IN_B>(src + tb * src_stride + (fb & mask) * C::IN_B);
+    const int64_t fo = odd ? fb - 1 : fa, to = fo >> row_shift;  // a pair lies in one row
+    slot = to < g.num_tokens ? g.slots[to] : int64_t(-1);
+    io = fo & mask;
+  }
+  const QScale qs = make_qscale_uniform(scale_p ? *scale_p : 1.0f);
+  const u32x2 qa = C::apply(va, qs), qb = C::apply(vb, qs);
+  // even lanes send vector 64 + l and take the neighbour's l + 1; odd lanes the reverse
+  const u32x2 send = odd ? qa : qb, keep = odd ? qb : qa;
+  constexpr int kXor1 = 0xB1;  // quad_perm [1,0,3,2]
+  const u32x2 got = {uint32_t(__builtin_amdgcn_update_dpp(0, int(send[0]), kXor1, 0xF, 0xF, false)),
+                     uint32_t(__builtin_amdgcn_update_dpp(0, int(send[1]), kXor1, 0xF, 0xF, false))};
+  const u32x4 w = odd ? u32x4{got[0], got[1], keep[0], keep[1]} : u32x4{keep[0], keep[1], got[0], got[1]};
+  if (slot >= 0 && slot < g.num_slots)
+    vstore_nt<16>(dst + (slot >> g.bs_shift) * blk_stride + (slot & (g.block_size - 1)) * page_stride + dst_off +
+                      io * C::OUT_B, w);
+}
+
+template <class C>
+bool launch_quant_pairs(const ScatterGeom& g, const ScatterPart& p0, const ScatterPart& p1, hipStream_t st,
+                        int* status) {
+  if constexpr (C::IN_B == 16 && C::OUT_B == 8) {
+    const int sh = log2_exact(p0.seg_vecs);
+    const uint64_t out[8] = {uint64_t(uintptr_t(p0.dst)), uint64_t(p0.blk_stride), uint64_t(p0.page_stride),
+                             uint64_t(p0.dst_off),        uint64_t(uintptr_t(p1.dst)), uint64_t(p1.blk_stride),
+                             uint64_t(p1.page_stride),    uint64_t(p1.dst_off)};
+    if (g.nparts != 2 || sh < 1 || p1.seg_vecs != p0.seg_vecs || common_align(out, 8, 16) < 16) return false;
+    // Rows of 64 vectors and more leave no lane idle either way: there the
+    // larger appends, bound by HBM, stay with a token per wave.
+    if (sh >= 6 && g.num_tokens << sh > int64_t(1) << 19) return false;
+    const int64_t waves = 2 * ceil_div(g.num_tokens << sh, 2 * kWave);
+    if (ceil_div(waves, 4) > INT32_MAX) return false;
+    const dim3 grid(unsigned(ceil_div(waves, 4)));
+    if (sh >= 7)
+      hipLaunchKernelGGL((quant_pair_scatter_kernel<C, true>), grid, dim3(256), 0, st, g, p0, p1, sh);
+    else
+      hipLaunchKernelGGL((quant_pair_scatter_kernel<C, false>), grid, dim3(256), 0, st, g, p0, p1, sh);
+    *status = check_launch("quant_pair_scatter_kernel launch");
+    return true;
+  }
+  return false;
+}
+
 bool part_flat(const ScatterPart& p, int out_b) { return p.nseg == 1 && p.inner_stride == out_b; }
 
 // fin: finish the amax scales in the append's own waves (the small kernel
@@ -502,6 +591,7 @@ int launch_scatter(const ScatterGeom& g, const ScatterPart& p0, const ScatterPar
   if (sh.ch == 1) return launch_scatter_shape<C, 1, 1, true, 1>(g, p0, p1, sh.slice_shift, st);
   int packed_status;
   if (launch_packed_rows<C>(g, p0, p1, st, &packed_status)) return packed_status;
+  if (launch_quant_pairs<C>(g, p0, p1, st, &packed_status)) return packed_status;
   // A quantizing append gets one token per wave and one vector per lane (a row
   // longer than 64 vectors loops): 32768 prefill tokens of config 2's geometry
   // 38.6 us against 39.8 at two tokens per wave, 40.9 at two vectors per lane
