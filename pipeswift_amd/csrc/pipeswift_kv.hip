@@ -760,6 +760,67 @@ __global__ void __launch_bounds__(256) paged_gather_kernel(GatherGeom g) {
   }
 }
 
+// Rows shorter than a wave (a power of two of at most 32 vectors of 16 output
+// bytes): the lanes pack 64 >> row_shift tokens into every load, CH loads a
+// wave, so that no lane idles.  The wave's first token finds its sequence as
+// above; a lane whose token lies past the end of that sequence walks on from
+// there.  Table entries load for all tokens before the first row does.
+// K and V of 128 elements a head, 6 sequences of up to 60000 tokens, us, four
+// tokens a wave against this with one, two and four loads a wave: FP8 to bf16,
+// 1 head 46.7 / 28.9 / 24.7 / 24.9, 2 heads 49.2 / 52.3 / 44.4 / 43.2 (of up
+// to 4000 tokens 6.5 / 5.7 / 5.7 / 7.8); bf16, 1 head 36.1 / 24.2 / 22.2 /
+// 27.8.
+template <class C, int CH, bool POW2>
+__global__ void __launch_bounds__(256) packed_gather_kernel(GatherGeom g, int row_shift) {
+  const int lane = threadIdx.x & (kWave - 1);
+  const int64_t half = gridDim.x >> 1;
+  const int part = g.nparts == 2 && int64_t(blockIdx.x) >= half ? 1 : 0;
+  const int per = kWave >> row_shift;  // tokens per load
+  const int64_t t0 = ((int64_t(blockIdx.x) - part * half) * 4 +
+                      __builtin_amdgcn_readfirstlane(int(threadIdx.x) / kWave)) * (CH * per);
+  const char* src = part ? g.src1 : g.src0;
+  char* dst = part ? g.dst1 : g.dst0;
+  QScale qs;
+  qs.s = g.scale ? *g.scale : 1.0f;
+  qs.r = 0.0f;
+  qs.fast = false;
+  qs.neg = 0u;
+  int64_t b0[1], pos0[1], cu0;
+  find_rows<1>(g.cu, g.starts, g.batch, t0, lane, b0, pos0, cu0);
+  const int64_t end = g.cu[b0[0] < g.batch ? b0[0] + 1 : g.batch];
+  const int vec = lane & ((1 << row_shift) - 1);
+  int64_t blk[CH], off[CH];
+  bool wr[CH];
+#pragma unroll
+  for (int c = 0; c < CH; ++c) {
+    const int64_t t = t0 + c * per + (lane >> row_shift);
+    int64_t b = b0[0], p = pos0[0] + (t - t0);
+    if (b < g.batch && t >= end) {
+      do ++b; while (b < g.batch && t >= int64_t(g.cu[b + 1]));
+      if (b < g.batch) p = (g.starts ? int64_t(g.starts[b]) : 0) + t - int64_t(g.cu[b]);
+    }
+    wr[c] = t < g.num_tokens && b < g.batch && t >= cu0;
+    // p < 2^32 where it is used: a start and a distance in int32 each
+    const uint32_t q = uint32_t(p);
+    const uint32_t page = POW2 ? q >> g.bs_shift : q / uint32_t(g.block_size);
+    off[c] = q - page * uint32_t(g.block_size);
+    blk[c] = -1;
+    if (wr[c] && p >= 0 && int64_t(page) < g.bt_stride) blk[c] = g.block_table[b * g.bt_stride + page];
+  }
+  typename C::In v[CH];
+#pragma unroll
+  for (int c = 0; c < CH; ++c) {
+    v[c] = typename C::In{};
+    if (blk[c] >= 0 && blk[c] < g.num_blocks)
+      v[c] = vload_nt<C::IN_B>(src + blk[c] * g.blk_stride + off[c] * g.page_stride + vec * C::IN_B);
+  }
+#pragma unroll
+  for (int c = 0; c < CH; ++c) {
+    const int64_t t = t0 + c * per + (lane >> row_shift);
+    if (wr[c]) vstore_nt<C::OUT_B>(dst + t * g.dst_stride + vec * C::OUT_B, C::apply(v[c], qs));
+  }
+}
+
 // Workgroups of `wpb` waves for chunks of `ch` tokens: the same number per
 // part (paged_gather_kernel splits the grid in halves between K and V).
 inline int64_t gather_grid(const GatherGeom& g, int ch, int wpb) {
@@ -789,7 +850,28 @@ void launch_gather_pow2(const GatherGeom& g, hipStream_t st) {
 }
 
 template <class C>
+bool launch_packed_gather(const GatherGeom& g, hipStream_t st) {
+  if constexpr (C::OUT_B == 16) {
+    // Rows of up to 256 cache bytes: bf16 rows of 512 are faster with four
+    // tokens a wave (6 x up to 60000 tokens 40.1 us against 41.6-45.9).  Below
+    // 4096 tokens the per-token waves, one token each, have the shorter chain.
+    const int sh = log2_exact(g.row_vecs);
+    if (sh < 0 || sh > 5 || g.row_vecs * C::IN_B > 256 || g.num_tokens < 4096 || g.block_size > INT32_MAX)
+      return false;
+    constexpr int CH = 2;
+    const dim3 grid(unsigned(ceil_div(ceil_div(g.num_tokens, CH * (kWave >> sh)), 4) * g.nparts));
+    if (g.bs_shift >= 0)
+      hipLaunchKernelGGL((packed_gather_kernel<C, CH, true>), grid, dim3(256), 0, st, g, sh);
+    else
+      hipLaunchKernelGGL((packed_gather_kernel<C, CH, false>), grid, dim3(256), 0, st, g, sh);
+    return true;
+  }
+  return false;
+}
+
+template <class C>
 int launch_gather(const GatherGeom& g, hipStream_t st) {
+  if (launch_packed_gather<C>(g, st)) return check_launch("packed_gather_kernel launch");
   if (g.bs_shift >= 0)
     launch_gather_pow2<C, true>(g, st);
   else
