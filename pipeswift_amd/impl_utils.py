@@ -24,22 +24,14 @@ def _layer_scale(scale, layer_idx):
     return scale if scale.numel() == 1 else scale[layer_idx: layer_idx + 1]
 
 
-def _layer(cache, layer_idx):
-    # select() is the same view as cache[layer_idx], without the parsing of a
-    # general index (1.7 against 2.3 us)
-    if type(cache) is torch.Tensor and type(layer_idx) is int:
-        return cache.select(0, layer_idx)
-    return cache[layer_idx]
-
-
 def append_kv_cache(key, value, kv_cache_info: KVCacheInfo = None, layer_idx: int = 0):
     if key.shape[0] == 0:
         return
     reshape_and_cache_flash(
         key,
         value,
-        _layer(kv_cache_info.kv_cache[0], layer_idx),
-        _layer(kv_cache_info.kv_cache[1], layer_idx),
+        kv_cache_info.kv_cache[0][layer_idx],
+        kv_cache_info.kv_cache[1][layer_idx],
         kv_cache_info.slot_mapping,
         _layer_scale(kv_cache_info.k_scale, layer_idx),
         _layer_scale(kv_cache_info.v_scale, layer_idx),

@@ -66,52 +66,45 @@ def reshape_and_cache_flash(
     assert key_cache.ndim == 4 and value_cache.ndim == 4
     assert key.is_cuda and value.is_cuda and slot_mapping.is_cuda
 
-    # The call's time is this function's, not the GPU's (a decode-sized append
-    # runs 2.5 us): each shape and stride tuple is read once, since torch builds
-    # it anew on every access, and one stride array serves both caches.
-    tokens, num_heads, head_size = key.shape
-    v_tokens, v_heads, v_size = value.shape
-    num_blocks, block_size, kc_heads, kc_size = key_cache.shape
-    vc_heads, vc_size = value_cache.shape[2:]
-    assert v_heads == num_heads
-    assert v_size == head_size
-    assert kc_heads == num_heads
-    assert kc_size == head_size
-    assert vc_heads == num_heads
-    assert vc_size == head_size
+    num_heads = key.shape[1]
+    head_size = key.shape[2]
+    assert value.shape[1] == num_heads
+    assert value.shape[2] == head_size
+    assert key_cache.shape[2] == num_heads
+    assert key_cache.shape[3] == head_size
+    assert value_cache.shape[2] == num_heads
+    assert value_cache.shape[3] == head_size
 
-    dtype, cache_dtype = key.dtype, key_cache.dtype
-    is_fp8 = cache_dtype == torch.float8_e4m3fn
-    assert is_fp8 or cache_dtype == dtype, (
-        f"kv cache dtype {cache_dtype} does not match key dtype {dtype}"
+    is_fp8 = key_cache.dtype == torch.float8_e4m3fn
+    assert is_fp8 or key_cache.dtype == key.dtype, (
+        f"kv cache dtype {key_cache.dtype} does not match key dtype {key.dtype}"
     )
-    assert value_cache.dtype == cache_dtype
-    assert value.dtype == dtype
+    assert value_cache.dtype == key_cache.dtype
+    assert value.dtype == key.dtype
 
     # The reference addresses V with key_cache's block, page and head strides
     # and value_cache's dim stride (reshape_and_cache.py:55-60, 121-127).  With
     # differing strides that writes outside value_cache, so it is rejected here.
-    kc = key_cache.stride()
-    vc = value_cache.stride()
-    assert vc[:3] == kc[:3], (
+    assert value_cache.stride()[:3] == key_cache.stride()[:3], (
         "value_cache must share key_cache's block/page/head strides "
-        f"({vc[:3]} vs {kc[:3]})"
+        f"({value_cache.stride()[:3]} vs {key_cache.stride()[:3]})"
     )
     device = key_cache.device
     assert key.device == device and value.device == device and value_cache.device == device
-    _check_slots(slot_mapping, min(tokens, v_tokens), device)
+    _check_slots(slot_mapping, min(key.shape[0], value.shape[0]), device)
     if not is_fp8:
         assert k_scale is None and v_scale is None, "k_scale/v_scale only apply to an fp8 cache"
     _check_scale(k_scale, device, "k_scale")
-    if v_scale is not k_scale:
-        _check_scale(v_scale, device, "v_scale")
+    _check_scale(v_scale, device, "v_scale")
 
-    kc_array = _lib.i64_array(kc)
+    kc = key_cache.stride()
+    vc = (kc[0], kc[1], kc[2], value_cache.stride(3))
+    n = slot_mapping.shape[0]
     status = lib().psk_reshape_and_cache(
         ptr(key), ptr(value), ptr(key_cache), ptr(value_cache), ptr(slot_mapping),
-        slot_mapping.shape[0], num_heads, head_size, block_size, num_blocks,
-        key.stride(0), value.stride(0), kc_array, kc_array if vc == kc else _lib.i64_array(vc),
-        dtype_code(dtype), dtype_code(cache_dtype), ptr(k_scale), ptr(v_scale),
+        n, num_heads, head_size, key_cache.shape[1], key_cache.shape[0],
+        key.stride(0), value.stride(0), _lib.i64_array(kc), _lib.i64_array(vc),
+        dtype_code(key.dtype), dtype_code(key_cache.dtype), ptr(k_scale), ptr(v_scale),
         stream_handle(device),
     )
     check(status, "reshape_and_cache_flash")
