@@ -763,7 +763,7 @@ __global__ void __launch_bounds__(256) paged_gather_kernel(GatherGeom g) {
 // Rows shorter than a wave (a power of two of at most 32 vectors of 16 output
 // bytes): the lanes pack 64 >> row_shift tokens into every load, CH loads a
 // wave, so that no lane idles.  The wave's first token finds its sequence as
-// above; a lane whose token lies past the end of that sequence walks on from
+// above; a lane whose token lies past the end of that sequence searches on from
 // there.  Table entries load for all tokens before the first row does.
 // K and V of 128 elements a head, 6 sequences of up to 60000 tokens, us, four
 // tokens a wave against this with one, two and four loads a wave: FP8 to bf16,
@@ -796,7 +796,8 @@ __global__ void __launch_bounds__(256) packed_gather_kernel(GatherGeom g, int ro
     const int64_t t = t0 + c * per + (lane >> row_shift);
     int64_t b = b0[0], p = pos0[0] + (t - t0);
     if (b < g.batch && t >= end) {
-      do ++b; while (b < g.batch && t >= int64_t(g.cu[b + 1]));
+      ++b;  // most often the next sequence holds it
+      if (b < g.batch && t >= int64_t(g.cu[b + 1])) b = sequence_from(g.cu, g.batch, b + 1, t);
       if (b < g.batch) p = (g.starts ? int64_t(g.starts[b]) : 0) + t - int64_t(g.cu[b]);
     }
     wr[c] = t < g.num_tokens && b < g.batch && t >= cu0;
