@@ -976,6 +976,37 @@ constexpr int kHeadWaves = 8;
 constexpr int kHeadRing = 2;
 
 
+// The record of a head from its P phase waves' states in LDS, each of those
+// waves writing every P-th 64 columns of it.  (One wave for all of them was a
+// serial chain: 16 query heads over one kv head, one sequence of 200 tokens 17.3
+// against 12.8 us, 32 of 4000 20.2 / 15.8.)
+template <int NG, int HG, int P>
+__device__ __forceinline__ void merge_phases(float* part, int G, int lane, int wave, const float (*s_acc)[NG][kHead],
+                                             const float (*s_m)[NG], const float (*s_l)[NG]) {
+  const int w0 = wave % HG, phase = wave / HG;  // the head's phase 0, and this wave's phase
+  for (int i = 64 * phase + lane; i < G * kHead; i += 64 * P) {
+    const int g = i / kHead, d = i % kHead;
+    float mx = s_m[w0][g];
+#pragma unroll
+    for (int p = 1; p < P; ++p) mx = __builtin_fmaxf(mx, s_m[w0 + HG * p][g]);
+    float v = 0.0f;
+#pragma unroll
+    for (int p = 0; p < P; ++p) v += s_acc[w0 + HG * p][g][d] * __builtin_amdgcn_exp2f(s_m[w0 + HG * p][g] - mx);
+    part[2 * G + i] = v;
+  }
+  if (phase == 0 && lane < G) {
+    const int g = lane;
+    float mx = s_m[w0][g];
+#pragma unroll
+    for (int p = 1; p < P; ++p) mx = __builtin_fmaxf(mx, s_m[w0 + HG * p][g]);
+    float sum = 0.0f;
+#pragma unroll
+    for (int p = 0; p < P; ++p) sum += s_l[w0 + HG * p][g] * __builtin_amdgcn_exp2f(s_m[w0 + HG * p][g] - mx);
+    part[g] = mx;
+    part[G + g] = sum;
+  }
+}
+
 // Merge this wave's token slots and, with P phases per head, the P waves of
 // each head through LDS; write head h's partial record rec_idx.
 template <int NG, int HG, int P>
@@ -1023,29 +1054,7 @@ __device__ __forceinline__ void write_partial_heads(const DecodeArgs& a, Softmax
       }
     }
     __syncthreads();
-    if (wave < HG) {  // phase 0 of head `wave` writes the merged record
-      for (int i = lane; i < G * kHead; i += 64) {
-        const int g = i / kHead, d = i % kHead;
-        float mx = s_m[wave][g];
-#pragma unroll
-        for (int p = 1; p < P; ++p) mx = __builtin_fmaxf(mx, s_m[wave + HG * p][g]);
-        float v = 0.0f;
-#pragma unroll
-        for (int p = 0; p < P; ++p) v += s_acc[wave + HG * p][g][d] * __builtin_amdgcn_exp2f(s_m[wave + HG * p][g] - mx);
-        part[2 * G + i] = v;
-      }
-      if (lane < G) {
-        const int g = lane;
-        float mx = s_m[wave][g];
-#pragma unroll
-        for (int p = 1; p < P; ++p) mx = __builtin_fmaxf(mx, s_m[wave + HG * p][g]);
-        float sum = 0.0f;
-#pragma unroll
-        for (int p = 0; p < P; ++p) sum += s_l[wave + HG * p][g] * __builtin_amdgcn_exp2f(s_m[wave + HG * p][g] - mx);
-        part[g] = mx;
-        part[G + g] = sum;
-      }
-    }
+    merge_phases<NG, HG, P>(part, G, lane, wave, s_acc, s_m, s_l);
   }
 }
 
@@ -1061,29 +1070,7 @@ __device__ __forceinline__ void write_partial_heads(const DecodeArgs& a, Softmax
   } else {
     stash_pv<NG>(st, s_acc, s_m, s_l, wave, lane);
     __syncthreads();
-    if (wave < HG) {  // phase 0 of head `wave` writes the merged record
-      for (int i = lane; i < G * kHead; i += 64) {
-        const int g = i / kHead, d = i % kHead;
-        float mx = s_m[wave][g];
-#pragma unroll
-        for (int p = 1; p < P; ++p) mx = __builtin_fmaxf(mx, s_m[wave + HG * p][g]);
-        float v = 0.0f;
-#pragma unroll
-        for (int p = 0; p < P; ++p) v += s_acc[wave + HG * p][g][d] * __builtin_amdgcn_exp2f(s_m[wave + HG * p][g] - mx);
-        part[2 * G + i] = v;
-      }
-      if (lane < G) {
-        const int g = lane;
-        float mx = s_m[wave][g];
-#pragma unroll
-        for (int p = 1; p < P; ++p) mx = __builtin_fmaxf(mx, s_m[wave + HG * p][g]);
-        float sum = 0.0f;
-#pragma unroll
-        for (int p = 0; p < P; ++p) sum += s_l[wave + HG * p][g] * __builtin_amdgcn_exp2f(s_m[wave + HG * p][g] - mx);
-        part[g] = mx;
-        part[G + g] = sum;
-      }
-    }
+    merge_phases<NG, HG, P>(part, G, lane, wave, s_acc, s_m, s_l);
   }
 }
 
