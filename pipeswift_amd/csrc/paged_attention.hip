@@ -968,8 +968,14 @@ __device__ __forceinline__ void seek_unit(const int32_t* pref, int num_seqs, int
 // each of eight workgroups on eight XCDs requesting its own slice: a
 // read-only probe of config 2's pages streams 6.9 TB/s that way against 5.9
 // for head slices.  Workgroup j * NHG + hg serves run j of head group hg
-// (NHG = Hkv / HG).  One long sequence takes it too: 131072 tokens of 8 kv
-// heads 53.7 us against 58.3 with a 4-wave workgroup per head and run.
+// (NHG = Hkv / HG).  One sequence takes it too: against a 4-wave workgroup per
+// head and run, us, query heads / kv heads:
+//   tokens     16          200         1000        4000        16000       131072
+//   32 / 8  10.4 / 11.0 10.9 / 11.6 11.2 / 12.7 14.3 / 14.0 18.1 / 17.6 51.3 / 56.7
+//   32 / 4  11.0 / 12.0 11.5 / 13.1 11.8 / 13.5 14.8 / 16.2 16.7 / 17.9 33.1 / 34.2
+//   8 / 2   10.3 / 11.6 10.8 / 12.8 11.0 / 12.9 12.7 / 14.0 13.0 / 17.6 21.1 / 24.8
+//   8 / 1   10.4 / 11.9 10.9 / 13.0 11.1 / 13.2 12.8 / 13.6 12.9 / 20.9 16.9 / 24.6
+//   16 / 1  11.1 / 12.6 11.6 / 13.7 11.7 / 13.7 13.8 / 14.5 14.0 / 22.5 18.0 / 26.6
 constexpr int kHeadWaves = 8;
 // LDS tile slots per wave.  At one workgroup per CU deeper rings cost no
 // occupancy, but measured slower on config 2: 227 us at three against 225.
@@ -1589,11 +1595,15 @@ int psk_paged_decode_attention(const void* q, int64_t q_tok_stride, int64_t q_he
   // sequence is expected to have, so that a wave's records take one round of
   // loads (the balanced schedule spreads runs / sequences + 1 on average; the
   // split schedule at most max_splits), at most kCombineMaxWaves.  Four rows
-  // per wave when one wave suffices, else one row per workgroup.
+  // per wave when one wave suffices, else one row per workgroup.  One sequence
+  // alone leaves anything from one record to all the runs', and the merge of
+  // the waves costs a short one more than a second round of loads costs a long
+  // one: with 8 waves against 16, 32 query heads over 8, 200 tokens 10.9 / 12.2
+  // us, 1000 11.2 / 12.7, 16000 18.1 / 18.1, 131072 51.3 / 51.2.
   const int64_t recs = runs > 0 ? runs / num_seqs + 1 : a.max_splits;
   const bool quad = recs <= combine_batch<4>();
   const int64_t waves = quad ? 1
-                             : std::max<int64_t>(1, std::min<int64_t>(kCombineMaxWaves,
+                             : std::max<int64_t>(1, std::min<int64_t>(num_seqs == 1 ? 8 : kCombineMaxWaves,
                                                                       ceil_div(recs, combine_batch<1>())));
   const int rows = quad ? 4 : 1;
   const dim3 grid2{unsigned(ceil_div(num_kv_heads * G, rows)), unsigned(num_seqs), 1u};
