@@ -141,15 +141,6 @@ __device__ __forceinline__ void load_query_as(const char* src, float qd, int d0,
   }
 }
 
-// prefill_runs.hip: a prefill step cut into equal runs, for at most
-// prefill_runs_fit() sequences and kv heads; `a` as the decode reader's, with
-// a.q_len the most query tokens of a sequence, a.heads at most 256.
-int64_t prefill_runs_wgs();    // workgroups of a step: the device's CUs (0 if unknown)
-int64_t prefill_runs_words();  // int32 words of its workspace, no initial contents needed
-bool prefill_runs_fit(int64_t num_seqs, int64_t num_kv_heads);
-int launch_prefill_runs(const DecodeArgs& a, int64_t num_seqs, int q_dtype, int out_dtype, int32_t* workspace,
-                        hipStream_t st);
-
 }  // namespace psk_detail
 
 #endif  // PSK_PAGED_ATTENTION_H

@@ -10,7 +10,7 @@
 #include <cmath>
 #include <type_traits>
 
-#include "paged_attention.h"
+#include "prefill_runs.h"
 
 using namespace psk_detail;
 
@@ -58,7 +58,7 @@ constexpr int kPfLoads = kPfKeys * 8 / kPfLoaders;  // 16-byte chunks of K (and 
 static_assert(kPfKeys % 32 == 0 && kPfLoads >= 1 && kPfLoads * kPfLoaders == kPfKeys * 8,
               "a stage is whole 32-key blocks, its chunks spread evenly over the loaders");
 
-constexpr int kPfSortMax = 1024;  // sequences the pre-pass orders by length (more: batch order)
+static_assert(kPfRows == kBlockRows && kPfThreads == kRunThreads, "the blocks of both prefill kernels are the same");
 
 struct PrefillArgs {
   DecodeArgs a;
@@ -69,62 +69,18 @@ struct PrefillArgs {
   int32_t narrow;         // K/V page and row strides below 2^32: offsets from 32 x 32-bit products
 };
 
-// The launch order of the query blocks, in one workgroup of 1024 threads:
-// sequences by decreasing length (the keys their last block reads; without
-// query tokens last), ties in batch order, then each sequence's blocks from
-// its last (the most keys, when causal) to its first.  Writes order[k] and
-// the exclusive prefix blocks[k] of ceil(n_b / tq) over launch positions,
-// blocks[num_seqs] = the total.  Past kPfSortMax sequences the batch order is
-// kept.
 __global__ void __launch_bounds__(1024) prefill_blocks_kernel(DecodeArgs a, int num_seqs, int tq, int32_t* blocks,
                                                               int32_t* order) {
-  __shared__ int32_t s_key[kPfSortMax];
-  __shared__ int32_t s_order[kPfSortMax];
-  __shared__ int32_t s_wave[16];
-  const int tid = int(threadIdx.x), lane = tid & 63, wave = tid >> 6;
-  const bool sorted = num_seqs <= kPfSortMax;
-  if (sorted) {
-    int key = -1;
-    if (tid < num_seqs) key = q_count(a, tid) > 0 ? max(a.seq_lens[tid], 0) : -1;
-    s_key[tid] = key;
-    __syncthreads();
-    if (tid < num_seqs) {
-      int rank = 0;
-      for (int j = 0; j < num_seqs; ++j) {
-        const int kj = s_key[j];
-        rank += (kj > key || (kj == key && j < tid)) ? 1 : 0;
-      }
-      s_order[rank] = tid;
+  __shared__ OrderLds lds;
+  if (num_seqs <= kOrderMax) {
+    const int b = int(threadIdx.x);
+    if (b < num_seqs) {
+      lds.n[b] = q_count(a, b);
+      lds.len[b] = max(a.seq_lens[b], 0);
     }
     __syncthreads();
   }
-  int carry = 0;
-  for (int c0 = 0; c0 < num_seqs; c0 += 1024) {
-    const int k = c0 + tid;
-    const int b = k < num_seqs ? (sorted ? s_order[k] : k) : 0;
-    const int nb = k < num_seqs ? (q_count(a, b) + tq - 1) / tq : 0;
-    int x = nb;  // inclusive prefix over the wave
-#pragma unroll
-    for (int o = 1; o < 64; o <<= 1) {
-      const int y = __shfl_up(x, o);
-      if (lane >= o) x += y;
-    }
-    if (lane == 63) s_wave[wave] = x;
-    __syncthreads();
-    int before = 0, total = 0;
-    for (int w = 0; w < 16; ++w) {
-      const int t = s_wave[w];
-      before += w < wave ? t : 0;
-      total += t;
-    }
-    if (k < num_seqs) {
-      blocks[k] = carry + before + x - nb;
-      order[k] = b;
-    }
-    carry += total;
-    __syncthreads();
-  }
-  if (tid == 0) blocks[num_seqs] = carry;
+  order_blocks<1024>(a, num_seqs, tq, blocks, order, lds);
 }
 
 // The launch position of query block u (blocks[0] = 0 <= u < blocks[num_seqs]):
@@ -171,16 +127,20 @@ __device__ __forceinline__ void store_row4<PSK_DTYPE_BF16>(char* dst, f32x4 v) {
   *reinterpret_cast<u32x2*>(dst) = u32x2{lo, hi};
 }
 
+struct StageLds {
+  u32x4 k[2][kPfKeys * 16];  // bf16 K rows, chunk c of key t at c ^ (t & 15)
+  u32x4 v[2][kPfKeys * 16];  // fp16 V rows, chunk c of key t at c ^ (2 (t & 7))
+};
+
+// One workgroup's query block, of `total`.
 template <int Q_DT, int OUT_DT>
-__global__ void __launch_bounds__(kPfThreads) __attribute__((amdgpu_waves_per_eu(2)))
-prefill_attention_kernel(PrefillArgs p) {
+__device__ __forceinline__ void attend_block(const PrefillArgs& p, int total, StageLds& lds) {
   const DecodeArgs& a = p.a;
-  __shared__ u32x4 s_k[2][kPfKeys * 16];  // bf16 K rows, chunk c of key t at c ^ (t & 15)
-  __shared__ u32x4 s_v[2][kPfKeys * 16];  // fp16 V rows, chunk c of key t at c ^ (2 (t & 7))
+  auto& s_k = lds.k;
+  auto& s_v = lds.v;
   const int lane = int(threadIdx.x) & 63;
   const int wave = __builtin_amdgcn_readfirstlane(int(threadIdx.x) >> 6);
   const int Hkv = a.num_kv_heads;
-  const int total = p.blocks[p.num_seqs];
   const int idx = int(blockIdx.x) / Hkv, h = int(blockIdx.x) - idx * Hkv;
   if (idx >= total) return;
   const int k = __builtin_amdgcn_readfirstlane(block_sequence(p.blocks, p.num_seqs, idx, lane));
@@ -512,36 +472,54 @@ prefill_attention_kernel(PrefillArgs p) {
   }
 }
 
-template <int Q_DT>
-void launch_prefill_q(const PrefillArgs& p, int out_dtype, dim3 grid, hipStream_t st) {
-  if (out_dtype == PSK_DTYPE_BF16)
-    hipLaunchKernelGGL((prefill_attention_kernel<Q_DT, PSK_DTYPE_BF16>), grid, dim3(kPfThreads), 0, st, p);
-  else
-    hipLaunchKernelGGL((prefill_attention_kernel<Q_DT, PSK_DTYPE_F32>), grid, dim3(kPfThreads), 0, st, p);
+template <int Q_DT, int OUT_DT>
+__global__ void __launch_bounds__(kPfThreads) __attribute__((amdgpu_waves_per_eu(2)))
+prefill_attention_kernel(PrefillArgs p) {
+  __shared__ StageLds lds;
+  attend_block<Q_DT, OUT_DT>(p, p.blocks[p.num_seqs], lds);
 }
 
-// Whether a step is cut into equal runs (prefill_runs.hip) instead of given a
-// workgroup per query block.  What decides is how a workgroup per block fills
-// the chip, from what the host knows: about total_q / tq blocks per kv head,
-// and sequences of at most `keys` keys (the block table's width).  Runs win
-// where the blocks are few and long: their splits, records and merge cost
-// about 25 us, which a step of short sequences does not get back.  Where the
-// blocks fill the chip several times over, or get shorter from a fresh
-// prompt's last block to its first and so fill each other's gaps, a workgroup
-// per block is the faster: on a full chip, which its power limits, the kernel
-// here takes 3-5 % less time per key.  Measured (us, runs / workgroup per
-// block; 32 query heads): 512 new tokens over 32768, 8 kv heads, 268 / 892;
-// 2 x 256 over 8192, 4 kv heads, 89 / 249; 4096 over six prefixes of 14k-45k,
-// 4 kv heads, 1400 / 1738; 128 over 4096, 43 / 127; 64 over 1000, 34 / 43;
-// fresh prompts of 2000 tokens 68 / 69, on one kv head of 8 query heads 42 /
-// 66, of 500 39 / 26, of 4000 164 / 140, of 8000 535 / 485, 8 x 500 63 / 54.
-bool use_runs(int64_t total_q, int64_t max_seqlen_q, int64_t num_seqs, int64_t num_kv_heads, int64_t tq, int64_t keys,
-              int64_t workspace_len) {
-  if (!prefill_runs_fit(num_seqs, num_kv_heads) || workspace_len < prefill_runs_words()) return false;
-  const int64_t wgs = ceil_div(total_q, tq) * num_kv_heads;  // workgroups, one per block (a sequence's last may be partial)
-  if (keys >= 4 * max_seqlen_q) return keys >= 1024 && wgs <= 4 * prefill_runs_wgs();
-  return keys >= 1536 && wgs <= prefill_runs_wgs();
+// After prefill_runs_kernel: the merge of its records where it took the step,
+// a workgroup per query block where it left it.
+template <int Q_DT, int OUT_DT>
+__global__ void __launch_bounds__(kPfThreads) __attribute__((amdgpu_waves_per_eu(2)))
+prefill_either_kernel(PrefillArgs p, RunSpace s) {
+  __shared__ StageLds lds;
+  static_assert(sizeof(MergeLds) <= sizeof(StageLds), "the stages hold the merge's scratch");
+  const int total = uniform(p.blocks[p.num_seqs]);
+  if (total < 0)
+    merge_records<OUT_DT>(p.a, p.tq, s, reinterpret_cast<MergeLds&>(lds));
+  else
+    attend_block<Q_DT, OUT_DT>(p, total, lds);
 }
+
+template <int Q_DT, int OUT_DT>
+void launch_prefill_out(const PrefillArgs& p, const RunSpace* s, dim3 grid, hipStream_t st) {
+  if (s)
+    hipLaunchKernelGGL((prefill_either_kernel<Q_DT, OUT_DT>), grid, dim3(kPfThreads), 0, st, p, *s);
+  else
+    hipLaunchKernelGGL((prefill_attention_kernel<Q_DT, OUT_DT>), grid, dim3(kPfThreads), 0, st, p);
+}
+
+template <int Q_DT>
+void launch_prefill_q(const PrefillArgs& p, const RunSpace* s, int out_dtype, dim3 grid, hipStream_t st) {
+  if (out_dtype == PSK_DTYPE_BF16) launch_prefill_out<Q_DT, PSK_DTYPE_BF16>(p, s, grid, st);
+  else launch_prefill_out<Q_DT, PSK_DTYPE_F32>(p, s, grid, st);
+}
+
+// What the host can tell of a step whose sequences have at most `keys` keys:
+// kBlocks where no length within the bound prefers the equal runs, kRuns where
+// all do (the longest sequence has its query tokens at least), else kEither.
+enum Route { kBlocks, kRuns, kEither };
+Route route(int64_t total_q, int64_t max_seqlen_q, int64_t num_seqs, int64_t num_kv_heads, int64_t tq, int64_t keys,
+            int64_t cus) {
+  const int64_t wgs = ceil_div(total_q, tq) * num_kv_heads;
+  if (num_seqs > kOrderMax || 2 * num_kv_heads > cus || !prefers_runs(keys, max_seqlen_q, wgs, cus)) return kBlocks;
+  return prefers_runs(std::min(keys, max_seqlen_q), max_seqlen_q, wgs, cus) ? kRuns : kEither;
+}
+
+// Words of workspace: the launch order, and the runs' part.
+int64_t order_words(int64_t num_seqs) { return 2 * num_seqs + 1; }
 
 }  // namespace
 
@@ -549,7 +527,7 @@ extern "C" {
 
 int64_t psk_paged_prefill_workspace_len(int64_t num_seqs) {
   if (num_seqs < 0) return PSK_E_ARG;
-  return std::max(2 * num_seqs + 1, prefill_runs_words());
+  return order_words(num_seqs) + (num_seqs <= kOrderMax ? prefill_runs_words() : 0);
 }
 
 int psk_paged_prefill_attention(const void* q, int64_t q_tok_stride, int64_t q_head_stride, int q_dtype,
@@ -586,9 +564,9 @@ int psk_paged_prefill_attention(const void* q, int64_t q_tok_stride, int64_t q_h
   if (!q || !k_cache || !v_cache || !k_strides || !v_strides || !block_table || !seq_lens || !out || !workspace)
     return fail(PSK_E_ARG, "NULL pointer");
   if (!std::isfinite(softmax_scale)) return fail(PSK_E_ARG, "softmax_scale is not finite");
-  if (workspace_len < 2 * num_seqs + 1)
+  if (workspace_len < order_words(num_seqs))
     return fail(PSK_E_WORKSPACE, "workspace of %lld words, need %lld", (long long)workspace_len,
-                (long long)(2 * num_seqs + 1));
+                (long long)order_words(num_seqs));
   const int qsz = dtype_size(q_dtype), osz = dtype_size(out_dtype);
   const uint64_t kv_align[8] = {uint64_t(uintptr_t(k_cache)), uint64_t(uintptr_t(v_cache)), uint64_t(k_strides[0]),
                                 uint64_t(k_strides[1]),       uint64_t(k_strides[2]),       uint64_t(v_strides[0]),
@@ -658,18 +636,29 @@ int psk_paged_prefill_attention(const void* q, int64_t q_tok_stride, int64_t q_h
                 (long long)num_kv_heads);
 
   hipStream_t st = static_cast<hipStream_t>(stream);
-  if (use_runs(total_q, max_seqlen_q, num_seqs, num_kv_heads, p.tq, block_table_width * block_size, workspace_len))
-    return launch_prefill_runs(a, num_seqs, q_dtype, out_dtype, workspace, st);
-  hipLaunchKernelGGL(prefill_blocks_kernel, dim3(1), dim3(1024), 0, st, a, int(num_seqs), int(p.tq), workspace,
-                     workspace + num_seqs + 1);
-  const int st1 = check_launch("prefill_blocks_kernel launch");
-  if (st1 != PSK_OK) return st1;
-  const dim3 grid{unsigned(max_blocks * num_kv_heads), 1u, 1u};
+  const int64_t cus = prefill_cus();
+  const Route r = workspace_len < order_words(num_seqs) + prefill_runs_words()
+                      ? kBlocks
+                      : route(total_q, max_seqlen_q, num_seqs, num_kv_heads, p.tq, block_table_width * block_size, cus);
+  RunSpace space;
+  int st1;
+  if (r != kBlocks) {
+    st1 = launch_prefill_runs(a, num_seqs, ceil_div(total_q, p.tq) * num_kv_heads, r == kRuns, q_dtype, out_dtype,
+                              workspace + order_words(num_seqs), workspace, workspace + num_seqs + 1, &space, st);
+  } else {
+    hipLaunchKernelGGL(prefill_blocks_kernel, dim3(1), dim3(1024), 0, st, a, int(num_seqs), int(p.tq), workspace,
+                       workspace + num_seqs + 1);
+    st1 = check_launch("prefill_blocks_kernel launch");
+  }
+  if (r == kRuns || st1 != PSK_OK) return st1;
+  // (kEither: a workgroup per CU for the merge, where the blocks are fewer)
+  const dim3 grid{unsigned(std::max(max_blocks * num_kv_heads, r == kEither ? cus : 1)), 1u, 1u};
+  const RunSpace* s = r == kEither ? &space : nullptr;
   switch (q_dtype) {
-    case PSK_DTYPE_FP8_E4M3FN: launch_prefill_q<PSK_DTYPE_FP8_E4M3FN>(p, out_dtype, grid, st); break;
-    case PSK_DTYPE_BF16: launch_prefill_q<PSK_DTYPE_BF16>(p, out_dtype, grid, st); break;
-    case PSK_DTYPE_F16: launch_prefill_q<PSK_DTYPE_F16>(p, out_dtype, grid, st); break;
-    default: launch_prefill_q<PSK_DTYPE_F32>(p, out_dtype, grid, st); break;
+    case PSK_DTYPE_FP8_E4M3FN: launch_prefill_q<PSK_DTYPE_FP8_E4M3FN>(p, s, out_dtype, grid, st); break;
+    case PSK_DTYPE_BF16: launch_prefill_q<PSK_DTYPE_BF16>(p, s, out_dtype, grid, st); break;
+    case PSK_DTYPE_F16: launch_prefill_q<PSK_DTYPE_F16>(p, s, out_dtype, grid, st); break;
+    default: launch_prefill_q<PSK_DTYPE_F32>(p, s, out_dtype, grid, st); break;
   }
   return check_launch("prefill_attention_kernel launch");
 }

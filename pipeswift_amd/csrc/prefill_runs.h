@@ -1,0 +1,285 @@
+// What the two prefill kernels share (prefill_attention.hip: a workgroup per
+// query block; prefill_runs.hip: the step cut into equal runs): which of them a
+// step takes, the launch order of the query blocks, and the merge of the
+// partial records that runs leave of the blocks they share.
+//
+// The host knows only how long a sequence can be (the block table's width) and
+// that the longest is no shorter than its query tokens.  Where that does not
+// settle the choice it is the device's, in two launches: prefill_runs_kernel
+// reads the lengths and either runs the step or leaves the blocks' launch
+// order, and prefill_either_kernel then merges the records or runs the blocks.
+
+#ifndef PSK_PREFILL_RUNS_H
+#define PSK_PREFILL_RUNS_H
+
+#include "paged_attention.h"
+
+namespace psk_detail {
+
+constexpr int kBlockRows = 256;        // rows of a query block: kBlockRows / heads query tokens of one kv head
+constexpr int kRunWaves = 8;           // waves of a workgroup, in both kernels
+constexpr int kRunThreads = kRunWaves * 64;
+constexpr int kOrderMax = 1024;        // sequences that are ordered by length (more: batch order)
+constexpr int kRunMaxWgs = 256;        // workgroups that share a step cut into runs, at most
+
+// Whether a step runs faster cut into equal runs than with a workgroup per
+// query block, from the longest sequence that has query tokens (`keys`), the
+// most query tokens of a sequence, the workgroups that its blocks are
+// (ceil(total_q / tq) per kv head) and the device's CUs.  Runs win where the
+// blocks are few and long: their splits, records and merge cost about 25 us,
+// which a step of short sequences does not get back.  Where the blocks fill the
+// chip several times over, or get shorter from a fresh prompt's last block to
+// its first and so fill each other's gaps, a workgroup per block is the faster:
+// on a full chip, which its power limits, that kernel takes 3-5 % less time per
+// key.  Increasing in `keys`, so a bound on the lengths decides some steps.
+// Measured, us, runs / workgroup per block, fresh prompts by query heads / kv
+// heads:
+//   tokens    250        500        1000       1400       2000       3000        4000       8000
+//   32 / 8  21.2/18.5  29.9/25.2  39.3/39.0  46.5/50.6  66.9/67.3  102.7/96.7  154/140    496/488
+//   32 / 4  22.1/18.2  29.5/25.4  37.5/39.5  49.0/51.2  69.7/68.4  103.6/95.7  155/137    498/487
+//   16 / 2  21.8/18.0  28.9/25.1  35.0/39.1  40.2/49.8  49.8/67.0   65.0/94.3  95.7/122   265/253
+//   8 / 2   21.1/18.3  28.8/24.7  32.0/38.1  33.8/49.4  40.9/65.8   48.5/93.0  61.3/120   148/231
+//   8 / 1   21.8/17.9  28.7/24.8  34.0/38.6  37.9/49.1  40.7/65.7   49.0/92.8  60.8/121   150/231
+// over a prefix (32 / 8): 64 tokens over 1000 33/42, 128 over 4096 42/126, 256
+// over 1000 35/47, 512 over 32768 264/923; six prompts of 500 beside a decode
+// of 20000 70/554; 32 / 4: seven of 600 over 20000 each 1208/2030.
+__host__ __device__ inline bool prefers_runs(int64_t keys, int64_t max_q, int64_t wgs, int64_t cus) {
+  if (keys >= 4 * max_q) return keys >= 1024 && wgs <= 4 * cus;
+  return keys >= 1536 && wgs <= cus;
+}
+
+// A value that is the same in every lane, in scalar registers.
+__device__ __forceinline__ int uniform(int v) { return __builtin_amdgcn_readfirstlane(v); }
+__device__ __forceinline__ int64_t uniform(int64_t v) {
+  const uint64_t lo = uint32_t(uniform(int(v))), hi = uint32_t(uniform(int(v >> 32)));
+  return int64_t(hi << 32 | lo);
+}
+
+// LDS of order_blocks: each sequence's query tokens and length (the caller's,
+// for at most kOrderMax sequences), and its scratch.
+struct OrderLds {
+  int32_t n[kOrderMax], len[kOrderMax], order[kOrderMax], wave[16];
+};
+
+// The launch order of the query blocks, by one workgroup of NT threads:
+// sequences by decreasing length (the keys their last block reads; without
+// query tokens last), ties in batch order, then each sequence's blocks from
+// its last (the most keys, when causal) to its first.  Writes order[k] and
+// the exclusive prefix blocks[k] of ceil(n_b / tq) over launch positions,
+// blocks[num_seqs] = the total.  Past kOrderMax sequences the batch order is
+// kept (and lds.n and lds.len not read).
+template <int NT>
+__device__ __forceinline__ void order_blocks(const DecodeArgs& a, int num_seqs, int tq, int32_t* blocks, int32_t* order,
+                                             OrderLds& lds) {
+  const int tid = int(threadIdx.x), lane = tid & 63, wave = tid >> 6;
+  const bool sorted = num_seqs <= kOrderMax;
+  if (sorted) {
+    for (int b = tid; b < num_seqs; b += NT) {
+      const int key = lds.n[b] > 0 ? lds.len[b] : -1;
+      int rank = 0;
+      for (int j = 0; j < num_seqs; ++j) {
+        const int kj = lds.n[j] > 0 ? lds.len[j] : -1;
+        rank += (kj > key || (kj == key && j < b)) ? 1 : 0;
+      }
+      lds.order[rank] = b;
+    }
+    __syncthreads();
+  }
+  int carry = 0;
+  for (int c0 = 0; c0 < num_seqs; c0 += NT) {
+    const int k = c0 + tid;
+    const int b = k < num_seqs ? (sorted ? lds.order[k] : k) : 0;
+    const int nb = k < num_seqs ? ((sorted ? lds.n[b] : q_count(a, b)) + tq - 1) / tq : 0;
+    int x = nb;  // inclusive prefix over the wave
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+      const int y = __shfl_up(x, o);
+      if (lane >= o) x += y;
+    }
+    if (lane == 63) lds.wave[wave] = x;
+    __syncthreads();
+    int before = 0, total = 0;
+    for (int w = 0; w < NT / 64; ++w) {
+      const int t = lds.wave[w];
+      before += w < wave ? t : 0;
+      total += t;
+    }
+    if (k < num_seqs) {
+      blocks[k] = carry + before + x - nb;
+      order[k] = b;
+    }
+    carry += total;
+    __syncthreads();
+  }
+  if (tid == 0) blocks[num_seqs] = carry;
+}
+
+// A partial record: per wave 16 x 64 lanes x 4 floats of O^T as the lanes hold
+// it, then 32 maxima and 32 sums.
+constexpr int64_t kRunSlab = 16 * 64 * 4 + 64;
+constexpr int64_t kRunRecord = kRunSlab * kRunWaves;
+
+// What run j left as a partial record in its slot: its block (b, i), if any,
+// and the sequence's query tokens.
+struct RunDesc {
+  int32_t valid, b, i, n;
+};
+
+// The runs' part of the workspace.
+struct RunSpace {
+  RunDesc* desc;     // of each run: [0] its first piece, [1] its last
+  float* records;    // 2 per run and kv head
+  int32_t max_runs;  // runs per kv head at most
+};
+
+template <int OUT_DT>
+__device__ __forceinline__ void store_cols4(char* dst, f32x4 v);
+template <>
+__device__ __forceinline__ void store_cols4<PSK_DTYPE_F32>(char* dst, f32x4 v) {
+  *reinterpret_cast<f32x4*>(dst) = v;
+}
+template <>
+__device__ __forceinline__ void store_cols4<PSK_DTYPE_BF16>(char* dst, f32x4 v) {
+  *reinterpret_cast<bf16x4*>(dst) = __builtin_convertvector(v, bf16x4);  // RNE
+}
+
+// Row lane % 32 of a wave's 32 of a block of ni query tokens from row `first`
+// of q: columns 32 d + 8 q + 4 (lane / 32) .. + 3 of O^T in o[4 (d - d0) + q]
+// for d0 <= d < d0 + ND, the sum lt and the maximum m, times vd to the output
+// and (with d0 = 0) to the lse.
+template <int OUT_DT, int ND>
+__device__ __forceinline__ void write_row(const DecodeArgs& a, int64_t first, int ni, int h, float vd, int wave, int lane,
+                                          int d0, const f32x4 (&o)[4 * ND], float m, float lt) {
+  const int G = a.heads;
+  const int r = wave * 32 + (lane & 31);
+  const int ti = r / G, g = r - ti * G;
+  if (ti >= ni) return;
+  const int64_t tok = first + ti;
+  const float inv = lt > 0.0f ? vd / lt : 0.0f;  // no key seen: zeros, lse = -inf
+  char* dst = a.out + tok * a.out_tok_stride + int64_t(h * G + g) * a.out_head_stride;
+  constexpr int kEsz = Elt<OUT_DT>::kSize;
+#pragma unroll
+  for (int c = 0; c < 4 * ND; ++c)
+    store_cols4<OUT_DT>(dst + (32 * (d0 + (c >> 2)) + 8 * (c & 3) + 4 * (lane >> 5)) * kEsz, o[c] * inv);
+  if (lane < 32 && d0 == 0 && a.lse)
+    a.lse[int64_t(h * G + g) * a.lse_head_stride + tok] =
+        lt > 0.0f ? (m + __builtin_log2f(lt)) * 0.6931471805599453f : -__builtin_inff();
+}
+
+// LDS of merge_records.
+struct MergeLds {
+  RunDesc first[kRunMaxWgs], last[kRunMaxWgs];
+  int32_t begin[kRunMaxWgs];  // the runs that begin a block they do not end
+  int32_t wave[kRunWaves];
+};
+
+// Merges the partial records of the blocks that several runs share, by all
+// workgroups of the launch (kRunThreads threads).  Run j's record in slot 1 is
+// the first of such a block, whose others are the first pieces of the runs that
+// follow.  A task is one wave's: 32 columns of the 32 rows of a wave of one
+// block and kv head, so that the wave's 4 KiB of a record are in flight at
+// once; the tasks of the blocks there are go round the launch's waves.
+template <int OUT_DT>
+__device__ __forceinline__ void merge_records(const DecodeArgs& a, int tq, const RunSpace& s, MergeLds& lds) {
+  const int tid = int(threadIdx.x), lane = tid & 63, wave = uniform(tid >> 6);
+  const int Hkv = a.num_kv_heads;
+  static_assert(kRunMaxWgs <= kRunThreads, "a run per thread");
+  const bool own = tid < s.max_runs;
+  RunDesc last{0, 0, 0, 0};
+  if (own) {
+    lds.first[tid] = s.desc[2 * tid];
+    last = s.desc[2 * tid + 1];
+    lds.last[tid] = last;
+  }
+  const uint64_t begins = __ballot(own && last.valid);
+  if (lane == 0) lds.wave[wave] = __popcll(begins);
+  __syncthreads();
+  int before = 0, total = 0;
+#pragma unroll
+  for (int w = 0; w < kRunWaves; ++w) {
+    const int t = lds.wave[w];
+    before += w < wave ? t : 0;
+    total += t;
+  }
+  if (own && last.valid) lds.begin[before + __popcll(begins & ((uint64_t(1) << lane) - 1))] = tid;
+  __syncthreads();
+  total = uniform(total);
+  const int tasks = total * Hkv * kRunWaves * 4;
+  for (int t = int(blockIdx.x) * kRunWaves + wave; t < tasks; t += int(gridDim.x) * kRunWaves) {
+    const int d0 = t & 3, row_wave = (t >> 2) & (kRunWaves - 1);
+    const int rest = t / (4 * kRunWaves);
+    const int at = rest / Hkv, h = rest - at * Hkv;
+    const int j = uniform(lds.begin[at]);
+    const int b = uniform(lds.last[j].b), i = uniform(lds.last[j].i);
+    const int ni = min(tq, uniform(lds.last[j].n) - i * tq);
+    if (row_wave * 32 >= ni * a.heads) continue;  // no query rows
+    const int64_t first = q_first(a, b) + i * tq;
+    const float vd = descale(a.vd, a.vd_b, a.vd_h, b, h);
+    // how many of the following runs' first pieces are of the same block
+    int n = 0;
+    for (int k = j + 1;; k += 64) {
+      const int jl = min(k + lane, s.max_runs - 1);
+      const RunDesc other = lds.first[jl];
+      const uint64_t same = __ballot(k + lane < s.max_runs && other.valid && other.b == b && other.i == i);
+      n += same == ~0ull ? 64 : __builtin_ctzll(~same);
+      if (same != ~0ull) break;
+    }
+    // record r of the block: run j's slot 1, then slot 0 of run j + r
+    auto record = [&](int r) {
+      return s.records + ((int64_t(j + r) * Hkv + h) * 2 + (r == 0 ? 1 : 0)) * kRunRecord + row_wave * kRunSlab;
+    };
+    // four records at a time, their maxima, sums and columns in flight together;
+    // past the last a record is read again with weight 0
+    constexpr int R = 4;
+    auto max_of = [&](int r) { return record(r)[4096 + (lane & 31)]; };
+    float m = max_of(0);
+#pragma unroll 4
+    for (int r = R; r <= n; ++r) m = __builtin_fmaxf(m, max_of(r));
+    float l = 0.0f;
+    f32x4 o[4];
+#pragma unroll
+    for (int c = 0; c < 4; ++c) o[c] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    for (int r0 = 0; r0 <= n; r0 += R) {
+      float rm[R], rl[R];
+      f32x4 x[R][4];
+#pragma unroll
+      for (int k = 0; k < R; ++k) {
+        const float* rec = record(min(r0 + k, n));
+        rm[k] = rec[4096 + (lane & 31)];
+        rl[k] = rec[4096 + 32 + (lane & 31)];
+#pragma unroll
+        for (int c = 0; c < 4; ++c) x[k][c] = *reinterpret_cast<const f32x4*>(rec + ((4 * d0 + c) * 64 + lane) * 4);
+      }
+      if (r0 == 0) {
+#pragma unroll
+        for (int k = 1; k < R; ++k) m = __builtin_fmaxf(m, rm[k]);
+      }
+#pragma unroll
+      for (int k = 0; k < R; ++k) {
+        if (r0 + k > n) break;
+        const float w = __builtin_amdgcn_exp2f(rm[k] - m);
+        l += rl[k] * w;
+#pragma unroll
+        for (int c = 0; c < 4; ++c) o[c] += x[k][c] * w;
+      }
+    }
+    write_row<OUT_DT, 1>(a, first, ni, h, vd, row_wave, lane, d0, o, m, l);
+  }
+}
+
+// prefill_runs.hip.  `a` as the decode reader's, with a.q_len the most query
+// tokens of a sequence, a.heads at most kBlockRows; for at most kOrderMax
+// sequences and prefill_cus() / 2 kv heads.
+int64_t prefill_cus();         // CUs of the device, at most kRunMaxWgs (0 if unknown)
+int64_t prefill_runs_words();  // int32 words of a RunSpace, no initial contents needed
+// A step cut into equal runs, with its merge: `sure`.  Else the first launch of
+// a step that may take either kernel (`wgs`: its blocks' workgroups, for
+// prefers_runs): where it does not run the step itself `blocks` and `order`
+// receive the launch order, else blocks[num_seqs] = -1.  Fills `space` from
+// `workspace`.
+int launch_prefill_runs(const DecodeArgs& a, int64_t num_seqs, int64_t wgs, bool sure, int q_dtype, int out_dtype,
+                        int32_t* workspace, int32_t* blocks, int32_t* order, RunSpace* space, hipStream_t st);
+
+}  // namespace psk_detail
+
+#endif  // PSK_PREFILL_RUNS_H

@@ -10,7 +10,7 @@
 #include <mutex>
 #include <type_traits>
 
-#include "paged_attention.h"
+#include "prefill_runs.h"
 
 using namespace psk_detail;
 
@@ -51,8 +51,9 @@ namespace {
 // of their 2.4 GHz rate): power.  Six prefixes of 14k-45k with 4096 new tokens,
 // 32 query heads over 4 kv heads: 1400 us (1130 TFLOP/s), against 1738 with a
 // workgroup per block; 512 new tokens over 32768: 268 against 892.
-constexpr int kPfWaves = 8;
+constexpr int kPfWaves = kRunWaves;
 constexpr int kPfRows = kPfWaves * 32;
+static_assert(kPfRows == kBlockRows, "the blocks of both prefill kernels are the same");
 constexpr int kPfKeys = 64;  // keys per LDS stage
 constexpr int kPfThreads = kPfWaves * 64;
 constexpr int kPfBufs = 3;                            // converted stages in LDS
@@ -75,24 +76,15 @@ static_assert(kPfKeys * 8 == kPfThreads, "every thread stages one 16-byte chunk 
 constexpr int64_t kPfCost = 384;
 constexpr int kPfSnap = 3;          // a run boundary this close (in stages) to a block's end moves there
 constexpr int64_t kPfMinRun = 512;  // least cost of a run
-constexpr int kPfScanMax = 1024;    // sequences at most: every workgroup scans their costs
-// A partial record: per wave 16 x 64 lanes x 4 floats of O^T as the lanes hold
-// it, then 32 maxima and 32 sums.
-constexpr int64_t kPfSlab = 16 * 64 * 4 + 64;
-constexpr int64_t kPfRecord = kPfSlab * kPfWaves;
-
-// What run j left as a partial record in its slot: its block (b, i), if any.
-struct PfDesc {
-  int32_t valid, b, i, unused;
-};
-
 struct RunArgs {
   DecodeArgs a;
-  PfDesc* desc;      // of each run: [0] its first piece, [1] its last
-  float* records;    // 2 per run and kv head
+  RunSpace s;
   int32_t num_seqs;
-  int32_t max_runs;  // runs per kv head at most
   int32_t tq;        // query tokens per block
+  int32_t wgs, cus;  // for prefers_runs
+  int32_t sure;      // the step is cut into runs whatever its lengths
+  int32_t* blocks;   // the launch order of the blocks, where they are not run here
+  int32_t* order;
 };
 
 // A sequence's blocks: nb of them, block i costs base + i * step.
@@ -103,10 +95,10 @@ struct PfSeq {
   __device__ __forceinline__ int64_t upto(int64_t i) const { return i * base + step * (i * (i - 1) / 2); }
 };
 
-__device__ __forceinline__ PfSeq pf_seq(const DecodeArgs& a, int tq, int b) {
+__device__ __forceinline__ PfSeq pf_seq(const DecodeArgs& a, int tq, int n, int len) {
   PfSeq s;
-  s.n = q_count(a, b);
-  s.len = max(a.seq_lens[b], 0);
+  s.n = n;
+  s.len = len;
   s.nb = (s.n + tq - 1) / tq;
   // causal: block i reads about len - n + (i + 1) tq keys; else all of them
   s.base = kPfCost + (a.causal ? int64_t(max(s.len - s.n, 0)) + tq : int64_t(s.len));
@@ -135,13 +127,6 @@ struct PfBlock {
   }
 };
 
-// A value that is the same in every lane, in scalar registers.
-__device__ __forceinline__ int uniform(int v) { return __builtin_amdgcn_readfirstlane(v); }
-__device__ __forceinline__ int64_t uniform(int64_t v) {
-  const uint64_t lo = uint32_t(uniform(int(v))), hi = uint32_t(uniform(int(v >> 32)));
-  return int64_t(hi << 32 | lo);
-}
-
 // The block that cost x (0 <= x < prefix[num_seqs]) falls in.
 __device__ __forceinline__ PfBlock pf_block(const RunArgs& p, const int64_t* prefix, int64_t x) {
   int lo = 0, hi = p.num_seqs - 1;  // the last sequence with prefix <= x (those without blocks share the next one's)
@@ -150,7 +135,7 @@ __device__ __forceinline__ PfBlock pf_block(const RunArgs& p, const int64_t* pre
     if (prefix[mid] <= x) lo = mid; else hi = mid - 1;
   }
   lo = uniform(lo);
-  const PfSeq s = pf_seq(p.a, p.tq, lo);
+  const PfSeq s = pf_seq(p.a, p.tq, q_count(p.a, lo), max(p.a.seq_lens[lo], 0));
   const int64_t before = lo > 0 ? int64_t(prefix[lo]) : 0;  // prefix[0] is not stored
   const int64_t y = x - before;
   int i = 0, last = s.nb - 1;  // the last block with upto(i) <= y
@@ -165,7 +150,7 @@ __device__ __forceinline__ PfBlock pf_block(const RunArgs& p, const int64_t* pre
 
 // Runs per kv head for total cost T.
 __device__ __forceinline__ int pf_runs(const RunArgs& p, int64_t T) {
-  return int(max(int64_t(1), min(int64_t(p.max_runs), T / kPfMinRun)));
+  return int(max(int64_t(1), min(int64_t(p.s.max_runs), T / kPfMinRun)));
 }
 
 // First cost of run j of M for total cost T: 0 for j = 0, T for j = M, and
@@ -174,25 +159,74 @@ __device__ __forceinline__ int64_t pf_run_start(int64_t T, int j, int M) {
   return (T * int64_t((uint32_t(j) << 16) / uint32_t(M))) >> 16;
 }
 
-// Cost prefix of the sequences (prefix[b + 1]: up to b), by the NT threads of
-// a workgroup.
+// What every workgroup finds out about the step's sequences first.
+struct PfStep {
+  bool take;  // the step is cut into runs
+  int64_t T;  // its cost
+};
+
+// Inclusive prefix over the wave.
+__device__ __forceinline__ int64_t wave_prefix(int64_t x, int lane) {
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) {
+    const int64_t y = __shfl_up(x, o);
+    if (lane >= o) x += y;
+  }
+  return x;
+}
+__device__ __forceinline__ int wave_longest(int keys) {
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) keys = max(keys, __shfl_xor(keys, o));
+  return uniform(keys);
+}
+
+// Whether the step is cut into runs, by the threads of a workgroup (the same
+// answer in every one; the launch that follows reads it): if so the cost prefix
+// of the sequences (prefix[b + 1]: up to b), else their query tokens and
+// lengths in `seqs`.  Up to 64 sequences every wave does it for itself, a
+// sequence a lane, without a barrier.
 template <int NT>
-__device__ __forceinline__ void pf_scan(const RunArgs& p, int64_t* prefix, int64_t* s_wave) {
+__device__ __forceinline__ PfStep pf_step(const RunArgs& p, int64_t* prefix, int64_t* s_wave, OrderLds& seqs) {
   const int tid = int(threadIdx.x), lane = tid & 63, wave = tid >> 6;
+  const DecodeArgs& a = p.a;
+  if (p.num_seqs <= 64) {
+    const bool in = lane < p.num_seqs;
+    const int n = in ? q_count(a, lane) : 0, len = in ? max(a.seq_lens[lane], 0) : 0;
+    if (!p.sure && !prefers_runs(wave_longest(n > 0 ? len : 0), a.q_len, p.wgs, p.cus)) {
+      if (in) {
+        seqs.n[lane] = n;
+        seqs.len[lane] = len;
+      }
+      return PfStep{false, 0};
+    }
+    const PfSeq s = pf_seq(a, p.tq, n, len);
+    const int64_t x = wave_prefix(in ? s.upto(s.nb) : 0, lane);
+    if (in) prefix[lane + 1] = x;  // the same from every wave
+    return PfStep{true, uniform(int64_t(__shfl(x, 63)))};
+  }
+  int keys = 0;
+  for (int b = tid; b < p.num_seqs; b += NT) {
+    const int n = q_count(a, b), len = max(a.seq_lens[b], 0);
+    seqs.n[b] = n;
+    seqs.len[b] = len;
+    if (n > 0) keys = max(keys, len);
+  }
+  keys = wave_longest(keys);
+  if (lane == 0) s_wave[wave] = keys;
+  __syncthreads();
+#pragma unroll
+  for (int w = 0; w < NT / 64; ++w) keys = max(keys, int(s_wave[w]));
+  if (!p.sure && !prefers_runs(uniform(keys), a.q_len, p.wgs, p.cus)) return PfStep{false, 0};
   int64_t carry = 0;
   for (int c0 = 0; c0 < p.num_seqs; c0 += NT) {
     const int b = c0 + tid;
     int64_t own = 0;
-    if (b < p.num_seqs) {
-      const PfSeq s = pf_seq(p.a, p.tq, b);
+    if (b < p.num_seqs) {  // (the lengths that this thread read)
+      const PfSeq s = pf_seq(a, p.tq, seqs.n[b], seqs.len[b]);
       own = s.upto(s.nb);
     }
-    int64_t x = own;  // inclusive prefix over the wave
-#pragma unroll
-    for (int o = 1; o < 64; o <<= 1) {
-      const int64_t y = __shfl_up(x, o);
-      if (lane >= o) x += y;
-    }
+    const int64_t x = wave_prefix(own, lane);
+    __syncthreads();  // the previous values of s_wave are read
     if (lane == 63) s_wave[wave] = x;
     __syncthreads();
     int64_t before = 0, total = 0;
@@ -203,44 +237,9 @@ __device__ __forceinline__ void pf_scan(const RunArgs& p, int64_t* prefix, int64
     }
     if (b < p.num_seqs) prefix[b + 1] = carry + before + x;
     carry += total;
-    __syncthreads();
   }
-}
-
-template <int OUT_DT>
-__device__ __forceinline__ void store_row4(char* dst, f32x4 v);
-template <>
-__device__ __forceinline__ void store_row4<PSK_DTYPE_F32>(char* dst, f32x4 v) {
-  *reinterpret_cast<f32x4*>(dst) = v;
-}
-template <>
-__device__ __forceinline__ void store_row4<PSK_DTYPE_BF16>(char* dst, f32x4 v) {
-  typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
-  *reinterpret_cast<bf16x4*>(dst) = __builtin_convertvector(v, bf16x4);  // RNE
-}
-
-// Row lane % 32 of a wave's 32: columns 32 d + 8 q + 4 (lane / 32) .. + 3 of
-// O^T in o[4 (d - d0) + q] for d0 <= d < d0 + ND, the sum lt and the maximum
-// m, to the output and (with d0 = 0) the lse.
-template <int OUT_DT, int ND>
-__device__ __forceinline__ void pf_write_row(const RunArgs& p, const PfBlock& k, int h, int wave, int lane, int d0,
-                                             const f32x4 (&o)[4 * ND], float m, float lt) {
-  const DecodeArgs& a = p.a;
-  const int G = a.heads;
-  const int r = wave * 32 + (lane & 31);
-  const int ti = r / G, g = r - ti * G;
-  const int i0 = k.i * p.tq;
-  if (ti >= min(p.tq, k.n - i0)) return;
-  const int64_t tok = q_first(a, k.b) + i0 + ti;
-  const float inv = lt > 0.0f ? descale(a.vd, a.vd_b, a.vd_h, k.b, h) / lt : 0.0f;  // no key seen: zeros, lse = -inf
-  char* dst = a.out + tok * a.out_tok_stride + int64_t(h * G + g) * a.out_head_stride;
-  constexpr int kEsz = Elt<OUT_DT>::kSize;
-#pragma unroll
-  for (int c = 0; c < 4 * ND; ++c)
-    store_row4<OUT_DT>(dst + (32 * (d0 + (c >> 2)) + 8 * (c & 3) + 4 * (lane >> 5)) * kEsz, o[c] * inv);
-  if (lane < 32 && d0 == 0 && a.lse)
-    a.lse[int64_t(h * G + g) * a.lse_head_stride + tok] =
-        lt > 0.0f ? (m + __builtin_log2f(lt)) * 0.6931471805599453f : -__builtin_inff();
+  __syncthreads();
+  return PfStep{true, uniform(carry)};
 }
 
 // LDS at a byte address
@@ -282,15 +281,22 @@ __global__ void __launch_bounds__(kPfThreads) __attribute__((amdgpu_waves_per_eu
 prefill_runs_kernel(RunArgs p) {
   const DecodeArgs& a = p.a;
   __shared__ __attribute__((aligned(1024))) char s_lds[kPfRaws * kPfRaw + kPfBufs * kPfStage];
-  __shared__ int64_t s_prefix[kPfScanMax + 1];
+  __shared__ int64_t s_prefix[kOrderMax + 1];  // every workgroup scans the sequences' costs
   __shared__ int64_t s_wave[kPfWaves];
   const int tid = int(threadIdx.x);
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int Hkv = a.num_kv_heads;
-  pf_scan<kPfThreads>(p, s_prefix, s_wave);
-  __syncthreads();
-  const int64_t T = uniform(s_prefix[p.num_seqs]);
+  OrderLds& seqs = *reinterpret_cast<OrderLds*>(s_lds);
+  static_assert(sizeof(OrderLds) <= sizeof(s_lds), "the stages hold it until the first one");
+  const PfStep found = pf_step<kPfThreads>(p, s_prefix, s_wave, seqs);
+  if (!found.take) {
+    __syncthreads();
+    if (blockIdx.x == 0) order_blocks<kPfThreads>(a, p.num_seqs, p.tq, p.blocks, p.order, seqs);
+    return;
+  }
+  if (blockIdx.x == 0 && tid == 0) p.blocks[p.num_seqs] = -1;
+  const int64_t T = found.T;
   const int M = uniform(pf_runs(p, T));
   // Workgroup w runs on XCD w % 8: a kv head's runs, in order, on as few XCDs
   // as there are for it, since neighbouring runs read the same keys.
@@ -300,14 +306,14 @@ prefill_runs_kernel(RunArgs p) {
     const int per = 8 / Hkv, xcd = w & 7;
     const int share = (M + per - 1) / per;
     h = xcd % Hkv;
-    j = (w >> 3) < share ? (xcd / Hkv) * share + (w >> 3) : p.max_runs;
+    j = (w >> 3) < share ? (xcd / Hkv) * share + (w >> 3) : p.s.max_runs;
   }
   // run j's partial records: slot 0 the one of its first block, unless it
   // begins that block; slot 1 of a block it begins and does not end (its last)
   if (w == 0)
-    for (int i = tid; i < 2 * (p.max_runs - M); i += kPfThreads) p.desc[2 * M + i].valid = 0;
+    for (int i = tid; i < 2 * (p.s.max_runs - M); i += kPfThreads) p.s.desc[2 * M + i].valid = 0;
   if (j >= M) return;
-  if (h == 0 && tid < 2) p.desc[2 * j + tid].valid = 0;
+  if (h == 0 && tid < 2) p.s.desc[2 * j + tid].valid = 0;
   if (T == 0) return;
   const int64_t x_begin = uniform(pf_run_start(T, j, M));
   const int64_t x_end = uniform(pf_run_start(T, j + 1, M));
@@ -724,12 +730,12 @@ prefill_runs_kernel(RunArgs p) {
       frag[c] = f32x4{o[c >> 2][4 * (c & 3)], o[c >> 2][4 * (c & 3) + 1], o[c >> 2][4 * (c & 3) + 2],
                       o[c >> 2][4 * (c & 3) + 3]};
     if (sa == 0 && sb == ns) {
-      pf_write_row<OUT_DT, 4>(p, k, h, wave, lane, 0, frag, m, lt);
+      write_row<OUT_DT, 4>(a, q_first(a, b) + i0, ni, h, descale(a.vd, a.vd_b, a.vd_h, b, h), wave, lane, 0, frag, m, lt);
     } else {
       const int slot = sa == 0 ? 1 : 0;
-      if (h == 0 && tid == 0) p.desc[2 * j + slot] = PfDesc{1, b, k.i, 0};
+      if (h == 0 && tid == 0) p.s.desc[2 * j + slot] = RunDesc{1, b, k.i, q_count(a, b)};
       if (busy) {
-        float* rec = p.records + ((int64_t(j) * Hkv + h) * 2 + slot) * kPfRecord + wave * kPfSlab;
+        float* rec = p.s.records + ((int64_t(j) * Hkv + h) * 2 + slot) * kRunRecord + wave * kRunSlab;
 #pragma unroll
         for (int c = 0; c < 16; ++c) *reinterpret_cast<f32x4*>(rec + (c * 64 + lane) * 4) = frag[c];
         if (lane < 32) {
@@ -743,60 +749,11 @@ prefill_runs_kernel(RunArgs p) {
   }
 }
 
-// Merges the partial records of the blocks that several runs share.  Workgroup
-// (run j, kv head h, w) serves the 32 rows of wave w of the block that run j
-// begins and does not end, whose other records are the first pieces of the
-// runs that follow; wave d of it serves columns 32 d .. + 31, so that each
-// wave's 4 KiB of a record are in flight at once and enough of them are.
-constexpr int kPfCombineWaves = 4;
+// The merge of a step that is cut into runs whatever its lengths.
 template <int OUT_DT>
-__global__ void __launch_bounds__(64 * kPfCombineWaves) prefill_combine_kernel(RunArgs p) {
-  const DecodeArgs& a = p.a;
-  const int lane = int(threadIdx.x) & 63;
-  const int d0 = uniform(int(threadIdx.x) >> 6);
-  const int wave = int(blockIdx.x) & (kPfWaves - 1);
-  const int rest = int(blockIdx.x) / kPfWaves;
-  const int Hkv = a.num_kv_heads;
-  const int j = rest / Hkv, h = rest - j * Hkv;
-  const PfDesc own = p.desc[2 * j + 1];
-  // how many of the following runs' first pieces are of the same block
-  const int jl = j + 1 + lane;
-  const PfDesc other = p.desc[2 * min(jl, p.max_runs - 1)];
-  if (!own.valid) return;
-  PfBlock k;
-  k.b = own.b;
-  k.i = own.i;
-  k.n = q_count(a, own.b);
-  if (wave * 32 >= min(p.tq, k.n - k.i * p.tq) * a.heads) return;  // no query rows
-  bool same = jl < p.max_runs && other.valid && other.b == own.b && other.i == own.i;
-  uint64_t others = __ballot(same);
-  int n = others == ~0ull ? 64 : __builtin_ctzll(~others);
-  for (int at = j + 65; n == at - j - 1; at += 64) {  // a block over more than 65 runs
-    const PfDesc more = p.desc[2 * min(at + lane, p.max_runs - 1)];
-    same = at + lane < p.max_runs && more.valid && more.b == own.b && more.i == own.i;
-    others = __ballot(same);
-    n += others == ~0ull ? 64 : __builtin_ctzll(~others);
-  }
-  // record r of the block: run j's slot 1, then slot 0 of run j + r
-  auto record = [&](int r) {
-    return p.records + ((int64_t(j + r) * Hkv + h) * 2 + (r == 0 ? 1 : 0)) * kPfRecord + wave * kPfSlab;
-  };
-  float m = record(0)[4096 + (lane & 31)];
-#pragma unroll 4
-  for (int r = 1; r <= n; ++r) m = __builtin_fmaxf(m, record(r)[4096 + (lane & 31)]);
-  float l = 0.0f;
-  f32x4 o[4];
-#pragma unroll
-  for (int c = 0; c < 4; ++c) o[c] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll 4
-  for (int r = 0; r <= n; ++r) {
-    const float* rec = record(r);
-    const float w = __builtin_amdgcn_exp2f(rec[4096 + (lane & 31)] - m);
-    l += rec[4096 + 32 + (lane & 31)] * w;
-#pragma unroll
-    for (int c = 0; c < 4; ++c) o[c] += *reinterpret_cast<const f32x4*>(rec + ((4 * d0 + c) * 64 + lane) * 4) * w;
-  }
-  pf_write_row<OUT_DT, 1>(p, k, h, wave, lane, d0, o, m, l);
+__global__ void __launch_bounds__(kRunThreads) prefill_merge_kernel(DecodeArgs a, int tq, RunSpace s) {
+  __shared__ MergeLds lds;
+  merge_records<OUT_DT>(a, tq, s, lds);
 }
 
 template <int Q_DT, bool GEN>
@@ -817,9 +774,13 @@ void launch_prefill(const RunArgs& p, int q_dtype, int out_dtype, dim3 grid, hip
   }
 }
 
-// Workgroups of a prefill step on the current device: one per CU (its LDS
-// stages and 256 registers a wave leave no room for a second).
-int64_t prefill_wgs() {
+}  // namespace
+
+namespace psk_detail {
+
+// One workgroup per CU (its LDS stages and 256 registers a wave leave no room
+// for a second).
+int64_t prefill_cus() {
   static std::mutex mu;
   static std::map<int, int64_t> cache;
   int dev = 0;
@@ -829,32 +790,29 @@ int64_t prefill_wgs() {
   if (it != cache.end()) return it->second;
   int cus = 0;
   if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) return 0;
-  cache[dev] = cus;
-  return cus;
+  cache[dev] = std::min(cus, kRunMaxWgs);
+  return cache[dev];
 }
 
-}  // namespace
+// Alignment to 16 bytes, the descriptors and the records.
+int64_t prefill_runs_words() { return 4 + 2 * kRunMaxWgs * (kRunRecord + int64_t(sizeof(RunDesc) / 4)); }
 
-namespace psk_detail {
-
-int64_t prefill_runs_wgs() { return prefill_wgs(); }
-
-int64_t prefill_runs_words() { return 4 + 2 * prefill_wgs() * (kPfRecord + int64_t(sizeof(PfDesc) / 4)); }
-
-bool prefill_runs_fit(int64_t num_seqs, int64_t num_kv_heads) {
-  return num_seqs <= kPfScanMax && 2 * num_kv_heads <= prefill_wgs();
-}
-
-int launch_prefill_runs(const DecodeArgs& a, int64_t num_seqs, int q_dtype, int out_dtype, int32_t* workspace,
-                        hipStream_t st) {
+int launch_prefill_runs(const DecodeArgs& a, int64_t num_seqs, int64_t wgs, bool sure, int q_dtype, int out_dtype,
+                        int32_t* workspace, int32_t* blocks, int32_t* order, RunSpace* space, hipStream_t st) {
   RunArgs p{};
   p.a = a;
   p.num_seqs = int32_t(num_seqs);
   p.tq = kPfRows / a.heads;
-  p.max_runs = int32_t(prefill_wgs() / a.num_kv_heads);
-  p.desc = reinterpret_cast<PfDesc*>((reinterpret_cast<uintptr_t>(workspace) + 15) & ~uintptr_t(15));
-  p.records = reinterpret_cast<float*>(p.desc + 2 * p.max_runs);
-  const dim3 grid{unsigned(p.max_runs * a.num_kv_heads), 1u, 1u};
+  p.wgs = int32_t(std::min<int64_t>(wgs, INT32_MAX));
+  p.cus = int32_t(prefill_cus());
+  p.sure = sure ? 1 : 0;
+  p.blocks = blocks;
+  p.order = order;
+  p.s.max_runs = p.cus / a.num_kv_heads;
+  p.s.desc = reinterpret_cast<RunDesc*>((reinterpret_cast<uintptr_t>(workspace) + 15) & ~uintptr_t(15));
+  p.s.records = reinterpret_cast<float*>(p.s.desc + 2 * p.s.max_runs);
+  *space = p.s;
+  const dim3 grid{unsigned(p.s.max_runs * a.num_kv_heads), 1u, 1u};
   // pages of a multiple of 8 keys whose rows lie within 32-bit offsets: a
   // wave's staged keys share a page
   const bool uniform_pages = a.block_size % 8 == 0 && a.k_row >= 0 && a.v_row >= 0 &&
@@ -862,13 +820,13 @@ int launch_prefill_runs(const DecodeArgs& a, int64_t num_seqs, int q_dtype, int 
   if (uniform_pages) launch_prefill<false>(p, q_dtype, out_dtype, grid, st);
   else launch_prefill<true>(p, q_dtype, out_dtype, grid, st);
   const int st1 = check_launch("prefill_runs_kernel launch");
-  if (st1 != PSK_OK) return st1;
-  const dim3 grid2{unsigned(p.max_runs * a.num_kv_heads * kPfWaves), 1u, 1u};
+  if (!sure || st1 != PSK_OK) return st1;
+  const dim3 grid2{unsigned(4 * p.s.max_runs * a.num_kv_heads), 1u, 1u};  // a task a wave where every run shares a block
   if (out_dtype == PSK_DTYPE_BF16)
-    hipLaunchKernelGGL((prefill_combine_kernel<PSK_DTYPE_BF16>), grid2, dim3(64 * kPfCombineWaves), 0, st, p);
+    hipLaunchKernelGGL((prefill_merge_kernel<PSK_DTYPE_BF16>), grid2, dim3(kRunThreads), 0, st, a, p.tq, p.s);
   else
-    hipLaunchKernelGGL((prefill_combine_kernel<PSK_DTYPE_F32>), grid2, dim3(64 * kPfCombineWaves), 0, st, p);
-  return check_launch("prefill_combine_kernel launch");
+    hipLaunchKernelGGL((prefill_merge_kernel<PSK_DTYPE_F32>), grid2, dim3(kRunThreads), 0, st, a, p.tq, p.s);
+  return check_launch("prefill_merge_kernel launch");
 }
 
 }  // namespace psk_detail

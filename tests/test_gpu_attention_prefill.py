@@ -40,10 +40,11 @@ _Q_NAMES = {torch.bfloat16: "bf16", torch.float16: "f16", torch.float32: "f32", 
 
 def _prefill_case(dev, seed, lens, counts, Hq, Hkv, ps, causal, descales=True, num_splits=0, spare_rows=0,
                   out_dtype=torch.float32, q_dtype=torch.bfloat16, path="entry", scale=128 ** -0.5, k_sign=1.0,
-                  bad_ids=False):
+                  bad_ids=False, wide=0):
     """One ragged step through ``path`` ("entry": flash_attn_varlen_func as
     the reference calls it; "prefill": paged_prefill_attention directly;
-    "chunks": the decode reader over chunks), checked against the oracle."""
+    "chunks": the decode reader over chunks), checked against the oracle.
+    ``wide``: keys the block table is as wide as."""
     g = torch.Generator().manual_seed(seed)
     B = len(lens)
     P = max(64, sum(-(-x // ps) for x in lens) + 8)
@@ -52,6 +53,8 @@ def _prefill_case(dev, seed, lens, counts, Hq, Hkv, ps, causal, descales=True, n
     fused[:, 1] = (torch.randn((P, ps, Hkv, 128), generator=g) * 2.0).to(torch.float8_e4m3fn)
     W = max(1, max(-(-x // ps) for x in lens))
     bt = torch.stack([torch.randperm(P, generator=g)[:W] for _ in range(B)]).to(torch.int32)
+    if wide > W * ps:
+        bt = torch.cat([bt, torch.randint(0, P, (B, -(-wide // ps) - W), generator=g, dtype=torch.int32)], 1)
     if bad_ids:  # missing pages inside the sequences: their rows read as zeros
         for b in range(B):
             used = -(-lens[b] // ps)

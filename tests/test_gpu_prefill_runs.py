@@ -12,6 +12,7 @@ import pytest
 import torch
 
 from pipeswift_amd import attention
+from tests import prefill_schedule as S
 from tests.test_gpu_attention_prefill import _prefill_case
 
 pytestmark = pytest.mark.gpu
@@ -80,7 +81,8 @@ def test_runs_in_a_graph(dev):
     graph = torch.cuda.CUDAGraph()
     with torch.cuda.graph(graph):
         call(out)
-    for n in (1500, 100, 2048, 81):
+    # (81, 100 and 200 keys take a workgroup per block, the others the runs)
+    for n in (1500, 100, 2048, 81, 1100, 200):
         lens.fill_(n)
         q.normal_(generator=g)
         out.zero_()
@@ -88,6 +90,63 @@ def test_runs_in_a_graph(dev):
         eager = call(torch.empty_like(out))
         torch.cuda.synchronize()
         assert torch.equal(out.view(torch.int16), eager.view(torch.int16)), f"replay at {n} keys"
+
+
+@pytest.mark.parametrize("B", [64, 65, 130, 700])
+@pytest.mark.parametrize("long", [True, False])
+def test_many_sequences(dev, B, long):
+    """As many sequences as a wave has lanes, and more than that and than a
+    workgroup has threads, empty ones among them (in keys, in queries), under a
+    table of 1100 keys: with a long sequence the step is cut into runs (two
+    rounds of the scan at 700), without one the device leaves the blocks in
+    launch order."""
+    counts = [(i * 7) % 5 for i in range(B)]
+    lens = [c + (i * 13) % 40 if i % 11 else 0 for i, c in enumerate(counts)]
+    counts[B // 2], lens[B // 2] = 6, 1100 if long else 70
+    counts[0] = counts[B - 1] = 0
+    assert S.takes_runs(counts, lens, 16, 2) == long
+    _prefill_case(dev, 1490 + B, lens, counts, 16, 2, 16, True, wide=1100)
+
+
+def _step(dev, counts, lens, Hq, Hkv, ps=16, seed=1500):
+    g = torch.Generator(device=dev).manual_seed(seed)
+    need = [-(-n // ps) for n in lens]
+    P = sum(need) + 1
+    kv = torch.randn(P, 2, ps, Hkv, 128, generator=g, device=dev).to(torch.float8_e4m3fn)
+    perm = torch.randperm(P, generator=g, device=dev).to(torch.int32)
+    bt = torch.zeros(len(lens), max(need), dtype=torch.int32, device=dev)
+    at = 0
+    for b, n in enumerate(need):
+        bt[b, :n] = perm[at:at + n]
+        at += n
+    q = torch.randn(sum(counts), Hq, 128, generator=g, device=dev).to(torch.bfloat16)
+    cu = torch.tensor(np.r_[0, np.cumsum(counts)], dtype=torch.int32, device=dev)
+    return q, kv, bt, cu, torch.tensor(lens, dtype=torch.int32, device=dev)
+
+
+@pytest.mark.parametrize("counts,prefixes,Hq,Hkv,runs", [
+    ([500], [0], 32, 8, False), ([250, 3], [0, 0], 32, 8, False), ([3000], [0], 32, 8, False),
+    ([500] * 8, [0] * 8, 32, 8, False), ([700, 40], [300, 500], 32, 4, False),
+    ([500, 1], [0, 9000], 32, 8, True), ([64], [1000], 32, 8, True), ([2000], [0], 8, 1, True),
+])
+def test_the_lengths_choose_the_kernel(dev, counts, prefixes, Hq, Hkv, runs):
+    """Not the block table's width: under a table of 32768 keys a step gives
+    the same bits, those of a workgroup per block where that is its kernel."""
+    lens = [c + p for c, p in zip(counts, prefixes)]
+    assert S.takes_runs(counts, lens, Hq, Hkv) == runs
+    q, kv, bt, cu, L = _step(dev, counts, lens, Hq, Hkv)
+    wide = torch.zeros(len(lens), 2048, dtype=torch.int32, device=dev)
+    wide[:, :bt.shape[1]] = bt
+
+    def call(table, **kw):
+        print(f"counts {counts} prefixes {prefixes}: table of {table.shape[1] * 16} keys {list(kw)}", flush=True)
+        return attention.paged_prefill_attention(q, kv[:, 0], kv[:, 1], table, L, cu, max(counts), 128 ** -0.5,
+                                                 **kw).view(torch.int16)
+
+    tight = call(bt)
+    blocks = call(bt, workspace=torch.empty(2 * len(lens) + 1, dtype=torch.int32, device=dev))
+    assert torch.equal(tight, blocks) != runs
+    assert torch.equal(call(wide), tight)
 
 
 def test_small_workspace_takes_a_workgroup_per_block(dev):
