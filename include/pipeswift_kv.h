@@ -388,10 +388,13 @@ int64_t psk_paged_decode_workspace_len(int64_t num_seqs, int64_t q_len, int64_t 
  * (num_q_heads / num_kv_heads) tokens of one kv head reads its keys once, in one
  * workgroup, or in several that share its keys where a step has too few blocks
  * to fill the device.  out rows (bf16 or f32) need 4-element alignment.
- * workspace: device int32, psk_paged_prefill_workspace_len(num_seqs) words for
- * the current device, no initial contents needed; from 2 num_seqs + 1 words up
- * a smaller one is taken, and the step then keeps a workgroup per block.  Two
- * launches.
+ * Which it is follows from the lengths: where the block table's width leaves it
+ * open, the device decides.  workspace: device int32, no initial contents
+ * needed; psk_paged_prefill_workspace_len(num_seqs) words suffice for any step,
+ * psk_paged_prefill_step_workspace_len for a step whose sequences have at most
+ * max_seqlen_k keys (2 num_seqs + 1 where none of its lengths would share
+ * blocks, else about 68 MB).  From 2 num_seqs + 1 words up a smaller one is
+ * taken, and the step keeps a workgroup per block.  Two launches.
  */
 int psk_paged_prefill_attention(const void* q, int64_t q_tok_stride, int64_t q_head_stride, int q_dtype,
                                 const void* k_cache, const void* v_cache, const int64_t* k_strides,
@@ -408,6 +411,8 @@ int psk_paged_prefill_attention(const void* q, int64_t q_tok_stride, int64_t q_h
                                 int64_t workspace_len, void* stream);
 
 int64_t psk_paged_prefill_workspace_len(int64_t num_seqs);
+int64_t psk_paged_prefill_step_workspace_len(int64_t num_seqs, int64_t total_q, int64_t max_seqlen_q,
+                                             int64_t num_q_heads, int64_t num_kv_heads, int64_t max_seqlen_k);
 
 /*
  * FP8 MLA latent entries with one scale per 128-element tile (build-defined;

@@ -105,6 +105,7 @@ _SIGNATURES = {
          _vp, _i64, _vp],
     ),
     "psk_paged_prefill_workspace_len": (_i64, [_i64]),
+    "psk_paged_prefill_step_workspace_len": (_i64, [_i64] * 6),
     "psk_mla_fp8_tile_entry_bytes": (_i64, [_i64, _i64]),
     "psk_concat_and_cache_mla_fp8_tiles": (
         _int, [_vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _i64, _i64, _i64, _i64, _i64, _int, _vp],

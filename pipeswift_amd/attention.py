@@ -182,10 +182,22 @@ def paged_decode_attention(
 
 
 def prefill_workspace_words(num_seqs: int) -> int:
+    """int32 words that suffice for any prefill step of ``num_seqs`` sequences."""
     n = int(lib().psk_paged_prefill_workspace_len(num_seqs))
     if n < 0:
         check(n, "paged prefill workspace")
     return n
+
+
+def _prefill_workspace(words: int, least: int, device) -> torch.Tensor:
+    """A workspace of ``words``, or of the ``least`` that the step takes where
+    a GPU full of KV pages has no room for the partial results."""
+    try:
+        return torch.empty(words, dtype=torch.int32, device=device)
+    except torch.cuda.OutOfMemoryError:
+        if words <= least:
+            raise
+        return torch.empty(least, dtype=torch.int32, device=device)
 
 
 def paged_prefill_attention(
@@ -205,6 +217,7 @@ def paged_prefill_attention(
     causal: bool = True,
     workspace: Optional[torch.Tensor] = None,
     validate: bool = False,
+    max_seqlen_k: Optional[int] = None,
 ):
     """Attention of a prefill (or chunked-prefill) step over the paged FP8
     cache: ``paged_decode_attention``'s arguments and results (q~, scores,
@@ -219,8 +232,12 @@ def paged_prefill_attention(
     fp16 MFMA with V exact and P rounded once to fp16 (at most (2^-11 + K
     2^-25) max|V vd| more error for K keys), fp32 sums.
     ``workspace``: int32 of ``prefill_workspace_words(B)`` (about 68 MB, most
-    of it for the partial results; allocated when absent).  One of at least 2 B
-    + 1 words is taken too, and keeps a workgroup per block.  The ragged
+    of it for the partial results; when absent it is allocated, and only if
+    the step can have such blocks).  One of at least 2 B + 1 words is taken
+    too, and keeps a workgroup per block.  ``max_seqlen_k``: a bound on the
+    sequences' lengths where the caller has a closer one than the block
+    table's width, so that steps of short sequences go the shorter way
+    without asking the device (it only chooses between kernels).  The ragged
     layout contract, and ``validate``, are ``paged_decode_attention``'s."""
     assert q.is_cuda and k_cache.is_cuda and v_cache.is_cuda
     assert q.dim() == 3 and q.shape[2] == HEAD_DIM and q.stride(2) == 1, "q must be [T, Hq, 128] with unit last stride"
@@ -251,8 +268,12 @@ def paged_prefill_attention(
         out = torch.empty(TQ, Hq, HEAD_DIM, dtype=torch.bfloat16, device=device)
     assert out.dtype in _OUT_CODES and out.shape == (TQ, Hq, HEAD_DIM) and out.stride(2) == 1
     lse = torch.empty(Hq, TQ, dtype=torch.float32, device=device) if return_softmax_lse else None
+    keys = block_table.shape[1] * ps if max_seqlen_k is None else min(int(max_seqlen_k), block_table.shape[1] * ps)
+    need = int(lib().psk_paged_prefill_step_workspace_len(B, TQ, q_len, Hq, Hkv, keys))
+    if need < 0:
+        need = 2 * B + 1  # the call itself says what is wrong
     if workspace is None or workspace.numel() < 2 * B + 1:
-        workspace = torch.empty(prefill_workspace_words(B), dtype=torch.int32, device=device)
+        workspace = _prefill_workspace(need, 2 * B + 1, device)
     assert workspace.dtype == torch.int32 and workspace.device == device
     qd, qsb, qsh = _descale(q_descale, B, Hkv, device)
     kd, ksb, ksh = _descale(k_descale, B, Hkv, device)
@@ -264,7 +285,7 @@ def paged_prefill_attention(
         HEAD_DIM, ps, P, TQ, q_len, ptr(cu_seqlens_q), 1 if causal else 0, float(softmax_scale),
         ptr(qd), ptr(kd), ptr(vd), i64_array([qsb, qsh, ksb, ksh, vsb, vsh]), out.data_ptr(), out.stride(0),
         out.stride(1), _OUT_CODES[out.dtype], ptr(lse), TQ if lse is not None else 0, workspace.data_ptr(),
-        workspace.numel(), stream_handle(device),
+        min(workspace.numel(), need), stream_handle(device),
     )
     check(st, "paged_prefill_attention")
     return (out, lse) if return_softmax_lse else out
@@ -364,7 +385,7 @@ def flash_attn_varlen_func(
     routes through this same entry, attention.py:577-585, or more than 16
     query heads per kv head) the step runs ``paged_prefill_attention``, which
     reads each kv head's keys once per block of 256 query rows; ``num_splits``
-    and ``max_seqlen_k`` do not apply there."""
+    does not apply there, and ``max_seqlen_k`` only helps to choose the kernel."""
     assert seqused_k is not None and block_table is not None, "paged attention needs seqused_k and block_table"
     B = seqused_k.shape[0]
     assert cu_seqlens_q is not None and cu_seqlens_q.shape[0] == B + 1
@@ -375,7 +396,7 @@ def flash_attn_varlen_func(
     if q_len * max(group, 1) > MAX_ROWS:
         return paged_prefill_attention(q, k, v, block_table, seqused_k, cu_seqlens_q, q_len, softmax_scale,
                                        q_descale, k_descale, v_descale, out=out,
-                                       return_softmax_lse=return_softmax_lse, causal=causal)
+                                       return_softmax_lse=return_softmax_lse, causal=causal, max_seqlen_k=bound)
     # B rows of at most one token each: one per sequence, cu_seqlens_q is 0..B
     cu = None if q_len == 1 and q.shape[0] == B else cu_seqlens_q
     return paged_decode_attention(q, k, v, block_table, seqused_k, softmax_scale, q_descale, k_descale, v_descale,

@@ -530,6 +530,17 @@ int64_t psk_paged_prefill_workspace_len(int64_t num_seqs) {
   return order_words(num_seqs) + (num_seqs <= kOrderMax ? prefill_runs_words() : 0);
 }
 
+int64_t psk_paged_prefill_step_workspace_len(int64_t num_seqs, int64_t total_q, int64_t max_seqlen_q,
+                                             int64_t num_q_heads, int64_t num_kv_heads, int64_t max_seqlen_k) {
+  if (num_seqs < 0 || total_q < 0 || max_seqlen_q <= 0 || num_kv_heads <= 0 || num_q_heads <= 0 ||
+      num_q_heads % num_kv_heads || num_q_heads / num_kv_heads > kPfRows)
+    return PSK_E_ARG;
+  // (kRunMaxWgs: a device with fewer CUs takes the runs for no step that one with more does not)
+  const bool blocks = route(total_q, max_seqlen_q, num_seqs, num_kv_heads, kPfRows / (num_q_heads / num_kv_heads),
+                            max_seqlen_k, kRunMaxWgs) == kBlocks;
+  return order_words(num_seqs) + (blocks ? 0 : prefill_runs_words());
+}
+
 int psk_paged_prefill_attention(const void* q, int64_t q_tok_stride, int64_t q_head_stride, int q_dtype,
                                 const void* k_cache, const void* v_cache, const int64_t* k_strides,
                                 const int64_t* v_strides, const int32_t* block_table, int64_t block_table_stride,

@@ -130,8 +130,9 @@ def _step(dev, counts, lens, Hq, Hkv, ps=16, seed=1500):
     ([500, 1], [0, 9000], 32, 8, True), ([64], [1000], 32, 8, True), ([2000], [0], 8, 1, True),
 ])
 def test_the_lengths_choose_the_kernel(dev, counts, prefixes, Hq, Hkv, runs):
-    """Not the block table's width: under a table of 32768 keys a step gives
-    the same bits, those of a workgroup per block where that is its kernel."""
+    """Not the block table's width: under a table of 32768 keys, and with and
+    without a bound on the lengths, a step gives the same bits, those of a
+    workgroup per block where that is its kernel."""
     lens = [c + p for c, p in zip(counts, prefixes)]
     assert S.takes_runs(counts, lens, Hq, Hkv) == runs
     q, kv, bt, cu, L = _step(dev, counts, lens, Hq, Hkv)
@@ -147,6 +148,40 @@ def test_the_lengths_choose_the_kernel(dev, counts, prefixes, Hq, Hkv, runs):
     blocks = call(bt, workspace=torch.empty(2 * len(lens) + 1, dtype=torch.int32, device=dev))
     assert torch.equal(tight, blocks) != runs
     assert torch.equal(call(wide), tight)
+    assert torch.equal(call(wide, max_seqlen_k=max(lens)), tight)
+    out = attention.flash_attn_varlen_func(q, kv[:, 0], kv[:, 1], max(counts), cu, max(lens), L, wide,
+                                           softmax_scale=128 ** -0.5, causal=True)
+    assert torch.equal(out.view(torch.int16), tight)
+
+
+def test_workspace_only_where_it_is_used(dev):
+    """A fresh prompt allocates nothing for partial results; a step that may
+    leave them does; and on a GPU without room for them it still runs, with a
+    workgroup per block."""
+    counts, lens = [300], [300]
+    q, kv, bt, cu, L = _step(dev, counts, lens, 32, 8)
+    out = torch.empty(300, 32, 128, dtype=torch.bfloat16, device=dev)
+
+    def grown(table, seq_lens):
+        torch.cuda.synchronize()
+        torch.cuda.reset_peak_memory_stats()
+        before = torch.cuda.memory_allocated()
+        attention.paged_prefill_attention(q, kv[:, 0], kv[:, 1], table, seq_lens, cu, 300, out=out)
+        return torch.cuda.max_memory_allocated() - before
+
+    wide = torch.zeros(1, 512, dtype=torch.int32, device=dev)
+    wide[:, :bt.shape[1]] = bt
+    assert grown(bt, L) < 1 << 16
+    assert grown(wide, L) > 60 << 20
+    free, total = torch.cuda.mem_get_info()
+    torch.cuda.empty_cache()
+    try:
+        torch.cuda.set_per_process_memory_fraction((torch.cuda.memory_reserved() + (24 << 20)) / total)
+        assert grown(wide, L) < 1 << 20
+    finally:
+        torch.cuda.set_per_process_memory_fraction(1.0)
+    want = attention.paged_prefill_attention(q, kv[:, 0], kv[:, 1], bt, L, cu, 300)
+    assert torch.equal(out.view(torch.int16), want.view(torch.int16))
 
 
 def test_small_workspace_takes_a_workgroup_per_block(dev):

@@ -1,11 +1,14 @@
-"""CPU checks of the equal-run prefill schedule's model (tests/prefill_schedule.py):
-every stage of every block is one run's, and a shared block's records are one
-slot each of runs that follow each other (as the merge walks them)."""
+"""CPU checks of the equal-run prefill schedule's model (tests/prefill_schedule.py)
+and of the C rule that chooses between the prefill kernels: every stage of every
+block is one run's, a shared block's records are one slot each of runs that
+follow each other (as the merge walks them), and the workspace query asks for
+the partial results only where some length within the bound would use them."""
 
 import random
 
 import pytest
 
+from pipeswift_amd._lib import lib
 from tests import prefill_schedule as S
 
 SHAPES = [(32, 8), (32, 4), (8, 1), (16, 16), (6, 2), (256, 1), (8, 8), (128, 64)]
@@ -40,6 +43,43 @@ def test_every_stage_once_and_records_in_a_row(seed):
                 # the first of them in its run's slot of blocks it begins, the others in the other slot
                 assert all(p.sa > 0 for _, _, p in got[1:]) and all(k == 0 for _, k, _ in got[1:])
     assert not seen
+
+
+def _step_words(counts, Hq, Hkv, keys):
+    return lib().psk_paged_prefill_step_workspace_len(len(counts), sum(counts), max(counts), Hq, Hkv, keys)
+
+
+@pytest.mark.parametrize("counts,Hq,Hkv,keys,records", [
+    ([500], 32, 8, 500, False),          # a fresh prompt under a table of its own width
+    ([500], 32, 8, 32768, True),         # the same under a wide table: the device decides
+    ([2000], 32, 8, 2000, True),
+    ([8000], 32, 8, 1 << 20, True),      # 1000 workgroups: a long enough prefix would take the runs
+    ([8001 * 5], 32, 8, 1 << 20, False),  # past four blocks a CU no length does
+    ([100] * 1025, 32, 8, 4096, False),  # more sequences than the runs scan
+    ([64], 32, 8, 1023, False), ([64], 32, 8, 1024, True),
+    ([512], 512, 256, 65536, False),     # more kv heads than half the CUs
+])
+def test_workspace_follows_the_step(counts, Hq, Hkv, keys, records):
+    B = len(counts)
+    most = lib().psk_paged_prefill_workspace_len(B)
+    words = _step_words(counts, Hq, Hkv, keys)
+    assert words == (most if records else 2 * B + 1)
+    assert most >= 2 * B + 1
+
+
+def test_workspace_query_matches_the_rule():
+    """Against the rule itself over random steps, and refusals."""
+    r = random.Random(5)
+    for _ in range(3000):
+        Hq, Hkv = r.choice(SHAPES)
+        counts = [r.randint(1, r.choice([50, 900, 9000])) for _ in range(r.randint(1, 9))]
+        keys = r.choice([0, 500, 1023, 1024, 1535, 1536, r.randint(1, 70000)])
+        want = S.prefers_runs(keys, max(counts), S.wgs(counts, Hq, Hkv))
+        assert (_step_words(counts, Hq, Hkv, keys) > 2 * len(counts) + 1) == want
+    f = lib().psk_paged_prefill_step_workspace_len
+    for bad in [(-1, 5, 5, 32, 8, 9), (1, -5, 5, 32, 8, 9), (1, 5, 0, 32, 8, 9), (1, 5, 5, 30, 8, 9),
+                (1, 5, 5, 0, 8, 9), (1, 5, 5, 32, 0, 9), (1, 5, 5, 514, 2, 9)]:
+        assert f(*bad) < 0
 
 
 def test_a_bound_on_the_keys_decides_monotonically():
