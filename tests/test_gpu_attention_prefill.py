@@ -30,6 +30,7 @@ import torch
 
 from oracle import kv_oracle as O
 from pipeswift_amd import attention, fp8_kv
+from tests import prefill_schedule as S
 from tests.conftest import raw
 
 pytestmark = pytest.mark.gpu
@@ -40,11 +41,14 @@ _Q_NAMES = {torch.bfloat16: "bf16", torch.float16: "f16", torch.float32: "f32", 
 
 def _prefill_case(dev, seed, lens, counts, Hq, Hkv, ps, causal, descales=True, num_splits=0, spare_rows=0,
                   out_dtype=torch.float32, q_dtype=torch.bfloat16, path="entry", scale=128 ** -0.5, k_sign=1.0,
-                  bad_ids=False, wide=0):
+                  bad_ids=False, wide=0, holes=(), head_major=False):
     """One ragged step through ``path`` ("entry": flash_attn_varlen_func as
     the reference calls it; "prefill": paged_prefill_attention directly;
-    "chunks": the decode reader over chunks), checked against the oracle.
-    ``wide``: keys the block table is as wide as."""
+    "blocks": the same with a workspace of 2 B + 1 words, which keeps a
+    workgroup per query block; "chunks": the decode reader over chunks),
+    checked against the oracle.  ``wide``: keys the block table is as wide as;
+    ``holes``: (sequence, table entry) pairs of missing pages; ``head_major``:
+    cache views whose head stride is above the row stride."""
     g = torch.Generator().manual_seed(seed)
     B = len(lens)
     P = max(64, sum(-(-x // ps) for x in lens) + 8)
@@ -55,6 +59,9 @@ def _prefill_case(dev, seed, lens, counts, Hq, Hkv, ps, causal, descales=True, n
     bt = torch.stack([torch.randperm(P, generator=g)[:W] for _ in range(B)]).to(torch.int32)
     if wide > W * ps:
         bt = torch.cat([bt, torch.randint(0, P, (B, -(-wide // ps) - W), generator=g, dtype=torch.int32)], 1)
+    for k, (b, page) in enumerate(holes):
+        assert page < -(-lens[b] // ps)
+        bt[b, page] = -3 if k % 2 else P + 5
     if bad_ids:  # missing pages inside the sequences: their rows read as zeros
         for b in range(B):
             used = -(-lens[b] // ps)
@@ -70,6 +77,9 @@ def _prefill_case(dev, seed, lens, counts, Hq, Hkv, ps, causal, descales=True, n
     if k_sign != 1.0:
         ds[1] = ds[1] * k_sign
     fd = fused.to(dev)
+    if head_major:
+        fd = fd.transpose(2, 3).contiguous().transpose(2, 3)
+        assert fd.stride(3) > fd.stride(2)
     out = torch.full((TQ, Hq, 128), 7.0, dtype=out_dtype, device=dev)
     print(f"prefill case seed={seed} B={B} counts={list(counts)[:8]} Hq={Hq} Hkv={Hkv} ps={ps} causal={causal} "
           f"splits={num_splits} out={out_dtype} q={q_dtype} path={path}", flush=True)
@@ -82,9 +92,10 @@ def _prefill_case(dev, seed, lens, counts, Hq, Hkv, ps, causal, descales=True, n
         f = fp8_kv.attn_varlen_func()
         got, lse = f(q=q.to(dev), k=fd[:, 0], v=fd[:, 1], max_seqlen_q=int(max(counts)), cu_seqlens_q=cu_d,
                      max_seqlen_k=None, seqused_k=lens_d, block_table=bt.to(dev), num_splits=num_splits, **kw)
-    elif path == "prefill":
+    elif path in ("prefill", "blocks"):
+        ws = torch.empty(2 * B + 1, dtype=torch.int32, device=dev) if path == "blocks" else None
         got, lse = attention.paged_prefill_attention(q.to(dev), fd[:, 0], fd[:, 1], bt.to(dev), lens_d, cu_d,
-                                                     int(max(counts)), **kw)
+                                                     int(max(counts)), workspace=ws, **kw)
     else:
         got, lse = attention.chunked_prefill_attention(q.to(dev), fd[:, 0], fd[:, 1], int(max(counts)), cu_d, lens_d,
                                                        bt.to(dev), num_splits=num_splits, **kw)
@@ -116,7 +127,7 @@ def _prefill_case(dev, seed, lens, counts, Hq, Hkv, ps, causal, descales=True, n
 def _runs_prefill_kernel(path, counts, Hq, Hkv):
     """Whether the step runs the prefill kernel (flash_attn_varlen_func's
     routing: more than 16 query rows per kv head)."""
-    return path == "prefill" or (path == "entry" and max(counts) * max(Hq // Hkv, 1) > 16)
+    return path in ("prefill", "blocks") or (path == "entry" and max(counts) * max(Hq // Hkv, 1) > 16)
 
 
 def p_rounding_bound(keys, vmax):
@@ -142,14 +153,15 @@ def test_prefill_ragged(dev, Hq, Hkv, causal):
     _prefill_case(dev, 500 + Hq + Hkv + causal, lens, counts, Hq, Hkv, 16, causal)
 
 
+@pytest.mark.parametrize("path", ["entry", "blocks"])
 @pytest.mark.parametrize("ps", [16, 24, 64])
-def test_prefill_block_sizes(dev, ps):
+def test_prefill_block_sizes(dev, ps, path):
     """Other page sizes (24: page rows found by division), empty sequences
     and spare query rows past the last one; the decode reader over chunks of
     the same step (with an explicit split count) agrees as well."""
     counts = [40, 0, 130, 17, 0, 64]
     lens = [40 + 300, 12, 130, 17 + 5, 0, 64 + 1000]
-    a, vmax = _prefill_case(dev, 600 + ps, lens, counts, 32, 8, ps, True, spare_rows=5)
+    a, vmax = _prefill_case(dev, 600 + ps, lens, counts, 32, 8, ps, True, spare_rows=5, path=path)
     b, _ = _prefill_case(dev, 600 + ps, lens, counts, 32, 8, ps, True, spare_rows=5, path="chunks", num_splits=3)
     n = sum(counts)
     # each within its tolerance of the oracle, so within their sum of each other
@@ -195,30 +207,48 @@ def test_prefill_many_sequences(dev):
     _prefill_case(dev, 901, lens, counts, 16, 2, 16, True)
 
 
-def test_prefill_long_prefix(dev):
+@pytest.mark.parametrize("path", ["entry", "blocks"])
+def test_prefill_long_prefix(dev, path):
     """Config 3's shape at a smaller scale: 600 and 900 new tokens over
     prefixes of 2000 and 4000 cached tokens, 32 query heads over 4 kv heads,
     many stages per workgroup and the causal band across two of them."""
-    _prefill_case(dev, 902, [2600, 4900], [600, 900], 32, 4, 16, True)
+    _prefill_case(dev, 902, [2600, 4900], [600, 900], 32, 4, 16, True, path=path)
 
 
-def test_prefill_steep_scores_take_the_exact_redo(dev):
+@pytest.mark.parametrize("path", ["entry", "blocks"])
+def test_prefill_steep_scores_take_the_exact_redo(dev, path):
     """Scores spread over hundreds of binary orders of magnitude (softmax
-    scale 4): rows pass the prefill kernel's 2^15 headroom above the maximum
-    of their first 32 keys, so their workgroups recompute with exact row
-    maxima; results still match the float64 oracle."""
-    _prefill_case(dev, 903, [700, 90, 1500], [300, 90, 64], 32, 4, 16, True, scale=4.0)
+    scale 4): rows pass the 2^15 headroom above the maximum of their first 32
+    keys.  With a workgroup per block ("blocks", up to 24 stages) the
+    workgroups recompute with exact row maxima; the step cut into runs (the
+    entry's choice here) raises its maxima in place.  Both match the float64
+    oracle."""
+    lens, counts = [700, 90, 1500], [300, 90, 64]
+    assert S.takes_runs(counts, lens, 32, 4)
+    _prefill_case(dev, 903, lens, counts, 32, 4, 16, True, scale=4.0, path=path)
 
 
-def test_prefill_negative_score_scale(dev):
+@pytest.mark.parametrize("ps", [16, 24])
+def test_prefill_redo_of_a_fresh_prompt(dev, ps):
+    """The redo where the entry itself takes a workgroup per block: a prompt of
+    700 tokens, 11 stages a workgroup, masked and unmasked ones."""
+    assert not S.takes_runs([700], [700], 16, 2)
+    _prefill_case(dev, 909, [700], [700], 16, 2, ps, True, scale=4.0)
+
+
+@pytest.mark.parametrize("path", ["entry", "blocks"])
+def test_prefill_negative_score_scale(dev, path):
     """A negative k descale (the score scale's sign applied to q~, exactly)."""
-    _prefill_case(dev, 904, [400, 250], [120, 250], 16, 2, 16, True, k_sign=-1.0)
+    _prefill_case(dev, 904, [400, 250], [120, 250], 16, 2, 16, True, k_sign=-1.0, path=path)
+    _prefill_case(dev, 904, [2400], [64], 16, 2, 16, True, k_sign=-1.0, path=path)
 
 
-def test_prefill_missing_pages_read_as_zero_rows(dev):
+@pytest.mark.parametrize("path", ["entry", "blocks"])
+def test_prefill_missing_pages_read_as_zero_rows(dev, path):
     """Block-table entries outside [0, num_blocks) inside the sequences read
     as zero K and V rows (scores 0), as in the decode reader and the oracle."""
-    _prefill_case(dev, 905, [300, 200, 90], [100, 200, 40], 32, 8, 16, True, bad_ids=True)
+    _prefill_case(dev, 905, [300, 200, 90], [100, 200, 40], 32, 8, 16, True, bad_ids=True, path=path)
+    _prefill_case(dev, 905, [2300], [64], 32, 8, 16, True, holes=[(0, 1), (0, 40), (0, 143)], path=path)
 
 
 def test_prefill_page_stride_past_32_bits(dev):
@@ -300,12 +330,14 @@ def test_prefill_more_sequences_than_the_pre_pass_orders(dev):
     _prefill_case(dev, 907, lens, counts, 32, 4, 16, True)
 
 
-def test_prefill_bench_step_matches_decode_reader(dev):
+@pytest.mark.parametrize("blocks", [False, True])
+def test_prefill_bench_step_matches_decode_reader(dev, blocks):
     """The bench's prefill_attention step at full size (config 3 geometry:
     4096 query tokens over 6 sequences with 14k-45k cached keys, 32 query
     heads over 4 kv heads, random FP8 pages, per-tensor descales, the bench's
-    seeds): the prefill kernel against the decode reader over 2-token chunks
-    of the same step, float32 outputs.  Two independent kernels, each pinned
+    seeds): the prefill kernels (the equal runs that the step takes, and a
+    workgroup per block) against the decode reader over 2-token chunks
+    of the same step, float32 outputs.  Independent kernels, each pinned
     to the oracle at smaller sizes, agree to 1e-3 of the largest output."""
     import workloads
 
@@ -328,7 +360,9 @@ def test_prefill_bench_step_matches_decode_reader(dev):
     print(f"prefill bench step: N={N} keys={int(lens.sum())} P={P}", flush=True)
     a = torch.empty(N, Hq, D, dtype=torch.float32, device=dev)
     b = torch.empty_like(a)
-    attention.paged_prefill_attention(q, kc, vc, bt, lens, cu, maxq, D ** -0.5, None, kd, vd, out=a, causal=True)
+    ws = torch.empty(2 * len(cc.chunk) + 1, dtype=torch.int32, device=dev) if blocks else None
+    attention.paged_prefill_attention(q, kc, vc, bt, lens, cu, maxq, D ** -0.5, None, kd, vd, out=a, causal=True,
+                                      workspace=ws)
     attention.chunked_prefill_attention(q, kc, vc, maxq, cu, lens, bt, softmax_scale=D ** -0.5, causal=True,
                                         k_descale=kd, v_descale=vd, out=b)
     torch.cuda.synchronize()
