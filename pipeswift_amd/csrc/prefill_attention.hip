@@ -99,19 +99,6 @@ __device__ __forceinline__ int block_sequence(const int32_t* blocks, int num_seq
   return lo;
 }
 
-// Byte offsets, from a 16-key V tile of a stage, of this lane's four
-// transposed reads (pv_offsets without the ring slot's K half).
-__device__ __forceinline__ void pf_v_offsets(int lane, uint32_t (&off)[4]) {
-  const int r = lane & 15, s = lane >> 4;
-  const int tok = 4 * s + ((r >> 1) & 3);
-  const uint32_t row = uint32_t(1024 * (tok >> 3) + 128 * (tok & 7) + 8 * (r & 1));
-#pragma unroll
-  for (int k = 0; k < 4; ++k) {
-    const int c = 2 * k + (r >= 8 ? 1 : 0);
-    off[k] = row + uint32_t(16 * (c ^ (tok & 7)));
-  }
-}
-
 template <int OUT_DT>
 __device__ __forceinline__ void store_row4(char* dst, f32x4 v);
 template <>
