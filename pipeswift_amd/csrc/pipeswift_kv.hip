@@ -523,8 +523,13 @@ bool launch_quant_pairs(const ScatterGeom& g, const ScatterPart& p0, const Scatt
                              uint64_t(p1.page_stride),    uint64_t(p1.dst_off)};
     if (g.nparts != 2 || sh < 1 || p1.seg_vecs != p0.seg_vecs || common_align(out, 8, 16) < 16) return false;
     // Rows of 64 vectors and more leave no lane idle either way: there the
-    // larger appends, bound by HBM, stay with a token per wave.
+    // larger appends, bound by HBM, stay with a token per wave.  So do the
+    // smallest, which end with their waves' latency: rows of 64 vectors up to
+    // 2560 tokens (4 heads, us, a token per wave against this: 1024 tokens 2.05
+    // / 2.40, 2048 2.65 / 2.70, 2500 2.85 / 2.90, 3000 3.05 / 2.75), shorter rows
+    // at 1024 (2 heads 2.00 / 2.07; 1100 2.20 / 2.10).
     if (sh >= 6 && g.num_tokens << sh > int64_t(1) << 19) return false;
+    if (sh < 7 && g.num_tokens <= (sh == 6 ? 2560 : 1024)) return false;
     const int64_t waves = 2 * ceil_div(g.num_tokens << sh, 2 * kWave);
     if (ceil_div(waves, 4) > INT32_MAX) return false;
     const dim3 grid(unsigned(ceil_div(waves, 4)));

@@ -17,7 +17,11 @@ pytestmark = pytest.mark.gpu
 @pytest.mark.parametrize("tokens,heads,dim,ps,pad,dtype", [
     (1024, 8, 128, 16, 0, "bf16"),     # 128 vectors: a wave a row
     (1027, 16, 128, 16, 0, "f16"),     # 256: two waves a row
-    (1025, 4, 128, 64, 0, "bf16"),     # 64: two rows a wave, one left over
+    (1025, 4, 128, 64, 0, "bf16"),     # 64 up to 2560 tokens: the kernel without pairs
+    (2560, 4, 128, 64, 0, "bf16"),     # the same
+    (2561, 4, 128, 64, 0, "bf16"),     # 64: two rows a wave, one left over
+    (1024, 2, 128, 16, 0, "bf16"),     # 32 up to 1024 tokens: the kernel without pairs
+    (1025, 2, 128, 16, 0, "f16"),      # 32: four rows a wave, one left over
     (1039, 1, 128, 1, 0, "bf16"),      # 16: eight rows a wave
     (1155, 1, 16, 16, 0, "f16"),       # 2: sixty-four rows a wave
     (1024, 1, 8, 16, 0, "bf16"),       # one vector: the kernel without pairs
@@ -28,7 +32,7 @@ pytestmark = pytest.mark.gpu
 def test_prefill_fp8_append(dev, tokens, heads, dim, ps, pad, dtype):
     g = torch.Generator().manual_seed(tokens + heads)
     td = {"bf16": torch.bfloat16, "f16": torch.float16}[dtype]
-    P, row = 1400 // ps + 4, heads * dim
+    P, row = max(1400, tokens + 200) // ps + 4, heads * dim
     qkv = (torch.randn(tokens, 4 * row, generator=g) * 3).to(td)
     flat = qkv.view(-1)
     flat[torch.randint(0, flat.numel(), (64,), generator=g)] = float("nan")
