@@ -517,8 +517,13 @@ int psk_gather_mla_fp8_tiles(const void* kv_cache, void* dst, const int32_t* blo
   hipStream_t s = static_cast<hipStream_t>(stream);
   // The common entry, every vector of it 16 bytes wide: the kernel of several
   // tokens a wave.  Other sizes, f32 rows and entries on 4- or 8-byte
-  // boundaries stay with one token a wave, whose vectors follow the alignment.
-  if (out_dtype == PSK_DTYPE_BF16 && tiles == kTilesPerPass && 2 * rope_len == 128 && rv == 16) {
+  // boundaries stay with one token a wave, whose vectors follow the alignment,
+  // and so do small reads of few sequences, whose search is short and whose
+  // waves are few either way (us, one token a wave against two: one sequence of
+  // 512 tokens 2.15 / 2.33, 3072 2.80 / 2.93, 4096 3.10 / 3.10; 8 sequences,
+  // 1024 tokens 2.42 / 2.45, 2048 2.73 / 2.56; 32, 256 2.50 / 2.33).
+  if (out_dtype == PSK_DTYPE_BF16 && tiles == kTilesPerPass && 2 * rope_len == 128 && rv == 16 &&
+      (batch_size >= 8 || num_tokens >= 4096)) {
     const dim3 grid_rows(unsigned(ceil_div(num_tokens, kWaves * kRowsPerWave)));
     hipLaunchKernelGGL(tile_fp8_gather_rows_kernel, grid_rows, block, 0, s, g);
     return check_launch("tile_fp8_gather_rows_kernel launch");

@@ -15,10 +15,14 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("lens,ps,pad,starts", [
-    ([1], 64, 0, False),                       # one token: the wave's second has no row
-    ([2, 0, 5], 1, 0, True),                   # seven tokens: a workgroup that is not full
-    ([8], 64, 0, False),                       # a workgroup exactly
-    ([0, 3, 6, 0], 3, 0, True),                # pages of three: division instead of a shift
+    ([1], 64, 0, False),                       # few tokens and sequences: one token a wave
+    ([2, 0, 5], 1, 0, True), ([8], 64, 0, False), ([0, 3, 6, 0], 3, 0, True),
+    ([0, 1] + [0] * 6, 64, 0, False),          # 8 sequences, one token: the wave's second has no row
+    ([2, 0, 5] + [0] * 6, 1, 0, True),         # seven tokens: a workgroup that is not full
+    ([0] * 7 + [8], 64, 0, False),             # a workgroup exactly
+    ([0, 3, 6, 0] * 2, 3, 0, True),            # pages of three: division instead of a shift
+    ([2000, 2090], 128, 0, True),              # the last of one token a wave (4095 rows with the five beside them)
+    ([2000, 2091], 128, 0, True),              # 4096 rows: two tokens a wave
     ([1, 0, 2] * 30, 16, 0, True),             # 90 sequences: past the window of 64
     ([0] * 70 + [5] + [0] * 70 + [4], 4, 0, False),  # empty sequences fill whole windows
     ([3] * 63 + [1, 40], 16, 16, True),        # a wave across the end of the window; entries 672 bytes apart
