@@ -74,10 +74,7 @@ __global__ void __launch_bounds__(1024) prefill_blocks_kernel(DecodeArgs a, int 
   __shared__ OrderLds lds;
   if (num_seqs <= kOrderMax) {
     const int b = int(threadIdx.x);
-    if (b < num_seqs) {
-      lds.n[b] = q_count(a, b);
-      lds.len[b] = max(a.seq_lens[b], 0);
-    }
+    if (b < num_seqs) put_sequence(lds, b, q_count(a, b), max(a.seq_lens[b], 0));
     __syncthreads();
   }
   order_blocks<1024>(a, num_seqs, tq, blocks, order, lds);
@@ -475,7 +472,7 @@ prefill_either_kernel(PrefillArgs p, RunSpace s) {
   static_assert(sizeof(MergeLds) <= sizeof(StageLds), "the stages hold the merge's scratch");
   const int total = uniform(p.blocks[p.num_seqs]);
   if (total < 0)
-    merge_records<OUT_DT>(p.a, p.tq, s, reinterpret_cast<MergeLds&>(lds));
+    merge_records<OUT_DT, 8>(p.a, p.tq, s, reinterpret_cast<MergeLds&>(lds));
   else
     attend_block<Q_DT, OUT_DT>(p, total, lds);
 }

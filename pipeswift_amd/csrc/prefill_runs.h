@@ -12,6 +12,8 @@
 #ifndef PSK_PREFILL_RUNS_H
 #define PSK_PREFILL_RUNS_H
 
+#include <type_traits>
+
 #include "paged_attention.h"
 
 namespace psk_detail {
@@ -55,11 +57,15 @@ __device__ __forceinline__ int64_t uniform(int64_t v) {
   return int64_t(hi << 32 | lo);
 }
 
-// LDS of order_blocks: each sequence's query tokens and length (the caller's,
-// for at most kOrderMax sequences), and its scratch.
+// LDS of order_blocks: each sequence's query tokens and its length, -1 if it
+// has none of them (put_sequence, for at most kOrderMax sequences), and scratch.
 struct OrderLds {
-  int32_t n[kOrderMax], len[kOrderMax], order[kOrderMax], wave[16];
+  int32_t n[kOrderMax], key[kOrderMax], order[kOrderMax], wave[16];
 };
+__device__ __forceinline__ void put_sequence(OrderLds& lds, int b, int n, int len) {
+  lds.n[b] = n;
+  lds.key[b] = n > 0 ? len : -1;
+}
 
 // The launch order of the query blocks, by one workgroup of NT threads:
 // sequences by decreasing length (the keys their last block reads; without
@@ -67,7 +73,7 @@ struct OrderLds {
 // its last (the most keys, when causal) to its first.  Writes order[k] and
 // the exclusive prefix blocks[k] of ceil(n_b / tq) over launch positions,
 // blocks[num_seqs] = the total.  Past kOrderMax sequences the batch order is
-// kept (and lds.n and lds.len not read).
+// kept (and lds.n and lds.key not read).
 template <int NT>
 __device__ __forceinline__ void order_blocks(const DecodeArgs& a, int num_seqs, int tq, int32_t* blocks, int32_t* order,
                                              OrderLds& lds) {
@@ -75,10 +81,10 @@ __device__ __forceinline__ void order_blocks(const DecodeArgs& a, int num_seqs, 
   const bool sorted = num_seqs <= kOrderMax;
   if (sorted) {
     for (int b = tid; b < num_seqs; b += NT) {
-      const int key = lds.n[b] > 0 ? lds.len[b] : -1;
+      const int key = lds.key[b];
       int rank = 0;
       for (int j = 0; j < num_seqs; ++j) {
-        const int kj = lds.n[j] > 0 ? lds.len[j] : -1;
+        const int kj = lds.key[j];
         rank += (kj > key || (kj == key && j < b)) ? 1 : 0;
       }
       lds.order[rank] = b;
@@ -178,8 +184,10 @@ struct MergeLds {
 // the first of such a block, whose others are the first pieces of the runs that
 // follow.  A task is one wave's: 32 columns of the 32 rows of a wave of one
 // block and kv head, so that the wave's 4 KiB of a record are in flight at
-// once; the tasks of the blocks there are go round the launch's waves.
-template <int OUT_DT>
+// once; the tasks of the blocks there are go round the launch's workgroups,
+// then their waves, so that a few use every CU's share of the bandwidth.
+// R records' columns are in flight at a time.
+template <int OUT_DT, int R>
 __device__ __forceinline__ void merge_records(const DecodeArgs& a, int tq, const RunSpace& s, MergeLds& lds) {
   const int tid = int(threadIdx.x), lane = tid & 63, wave = uniform(tid >> 6);
   const int Hkv = a.num_kv_heads;
@@ -205,7 +213,7 @@ __device__ __forceinline__ void merge_records(const DecodeArgs& a, int tq, const
   __syncthreads();
   total = uniform(total);
   const int tasks = total * Hkv * kRunWaves * 4;
-  for (int t = int(blockIdx.x) * kRunWaves + wave; t < tasks; t += int(gridDim.x) * kRunWaves) {
+  for (int t = wave * int(gridDim.x) + int(blockIdx.x); t < tasks; t += int(gridDim.x) * kRunWaves) {
     const int d0 = t & 3, row_wave = (t >> 2) & (kRunWaves - 1);
     const int rest = t / (4 * kRunWaves);
     const int at = rest / Hkv, h = rest - at * Hkv;
@@ -228,22 +236,20 @@ __device__ __forceinline__ void merge_records(const DecodeArgs& a, int tq, const
     auto record = [&](int r) {
       return s.records + ((int64_t(j + r) * Hkv + h) * 2 + (r == 0 ? 1 : 0)) * kRunRecord + row_wave * kRunSlab;
     };
-    // four records at a time, their maxima, sums and columns in flight together;
-    // past the last a record is read again with weight 0
-    constexpr int R = 4;
+    // a batch of records at a time, their maxima, sums and columns in flight
+    // together (past the last a record is read again and not used): two where
+    // two runs share the block, else R
     auto max_of = [&](int r) { return record(r)[4096 + (lane & 31)]; };
-    float m = max_of(0);
-#pragma unroll 4
-    for (int r = R; r <= n; ++r) m = __builtin_fmaxf(m, max_of(r));
-    float l = 0.0f;
+    float m = max_of(0), l = 0.0f;
     f32x4 o[4];
 #pragma unroll
     for (int c = 0; c < 4; ++c) o[c] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-    for (int r0 = 0; r0 <= n; r0 += R) {
-      float rm[R], rl[R];
-      f32x4 x[R][4];
+    auto add = [&](auto batch_tag, int r0) {
+      constexpr int N = decltype(batch_tag)::value;
+      float rm[N], rl[N];
+      f32x4 x[N][4];
 #pragma unroll
-      for (int k = 0; k < R; ++k) {
+      for (int k = 0; k < N; ++k) {
         const float* rec = record(min(r0 + k, n));
         rm[k] = rec[4096 + (lane & 31)];
         rl[k] = rec[4096 + 32 + (lane & 31)];
@@ -252,16 +258,23 @@ __device__ __forceinline__ void merge_records(const DecodeArgs& a, int tq, const
       }
       if (r0 == 0) {
 #pragma unroll
-        for (int k = 1; k < R; ++k) m = __builtin_fmaxf(m, rm[k]);
+        for (int k = 1; k < N; ++k) m = __builtin_fmaxf(m, rm[k]);
       }
 #pragma unroll
-      for (int k = 0; k < R; ++k) {
+      for (int k = 0; k < N; ++k) {
         if (r0 + k > n) break;
         const float w = __builtin_amdgcn_exp2f(rm[k] - m);
         l += rl[k] * w;
 #pragma unroll
         for (int c = 0; c < 4; ++c) o[c] += x[k][c] * w;
       }
+    };
+    if (n == 1) {
+      add(std::integral_constant<int, 2>{}, 0);
+    } else {
+#pragma unroll 16
+      for (int r = R; r <= n; ++r) m = __builtin_fmaxf(m, max_of(r));
+      for (int r0 = 0; r0 <= n; r0 += R) add(std::integral_constant<int, R>{}, r0);
     }
     write_row<OUT_DT, 1>(a, first, ni, h, vd, row_wave, lane, d0, o, m, l);
   }

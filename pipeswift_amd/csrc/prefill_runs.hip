@@ -193,10 +193,7 @@ __device__ __forceinline__ PfStep pf_step(const RunArgs& p, int64_t* prefix, int
     const bool in = lane < p.num_seqs;
     const int n = in ? q_count(a, lane) : 0, len = in ? max(a.seq_lens[lane], 0) : 0;
     if (!p.sure && !prefers_runs(wave_longest(n > 0 ? len : 0), a.q_len, p.wgs, p.cus)) {
-      if (in) {
-        seqs.n[lane] = n;
-        seqs.len[lane] = len;
-      }
+      if (in) put_sequence(seqs, lane, n, len);
       return PfStep{false, 0};
     }
     const PfSeq s = pf_seq(a, p.tq, n, len);
@@ -207,8 +204,7 @@ __device__ __forceinline__ PfStep pf_step(const RunArgs& p, int64_t* prefix, int
   int keys = 0;
   for (int b = tid; b < p.num_seqs; b += NT) {
     const int n = q_count(a, b), len = max(a.seq_lens[b], 0);
-    seqs.n[b] = n;
-    seqs.len[b] = len;
+    put_sequence(seqs, b, n, len);
     if (n > 0) keys = max(keys, len);
   }
   keys = wave_longest(keys);
@@ -222,7 +218,7 @@ __device__ __forceinline__ PfStep pf_step(const RunArgs& p, int64_t* prefix, int
     const int b = c0 + tid;
     int64_t own = 0;
     if (b < p.num_seqs) {  // (the lengths that this thread read)
-      const PfSeq s = pf_seq(a, p.tq, seqs.n[b], seqs.len[b]);
+      const PfSeq s = pf_seq(a, p.tq, seqs.n[b], max(seqs.key[b], 0));
       own = s.upto(s.nb);
     }
     const int64_t x = wave_prefix(own, lane);
@@ -753,7 +749,7 @@ prefill_runs_kernel(RunArgs p) {
 template <int OUT_DT>
 __global__ void __launch_bounds__(kRunThreads) prefill_merge_kernel(DecodeArgs a, int tq, RunSpace s) {
   __shared__ MergeLds lds;
-  merge_records<OUT_DT>(a, tq, s, lds);
+  merge_records<OUT_DT, 4>(a, tq, s, lds);
 }
 
 template <int Q_DT, bool GEN>
