@@ -491,15 +491,25 @@ void launch_prefill_q(const PrefillArgs& p, const RunSpace* s, int out_dtype, di
   else launch_prefill_out<Q_DT, PSK_DTYPE_F32>(p, s, grid, st);
 }
 
-// What the host can tell of a step whose sequences have at most `keys` keys:
-// kBlocks where no length within the bound prefers the equal runs, kRuns where
-// all do (the longest sequence has its query tokens at least), else kEither.
+// What the host can tell of a step whose sequences have at most `keys` keys,
+// and its query tokens at least: kBlocks where no such lengths prefer the equal
+// runs, kRuns where all do, else kEither.
 enum Route { kBlocks, kRuns, kEither };
-Route route(int64_t total_q, int64_t max_seqlen_q, int64_t num_seqs, int64_t num_kv_heads, int64_t tq, int64_t keys,
-            int64_t cus) {
-  const int64_t wgs = ceil_div(total_q, tq) * num_kv_heads;
-  if (num_seqs > kOrderMax || 2 * num_kv_heads > cus || !prefers_runs(keys, max_seqlen_q, wgs, cus)) return kBlocks;
-  return prefers_runs(std::min(keys, max_seqlen_q), max_seqlen_q, wgs, cus) ? kRuns : kEither;
+Route route(int64_t total_q, int64_t max_q, int64_t num_seqs, int64_t num_kv_heads, int64_t tq, bool causal,
+            int64_t keys, int64_t cus) {
+  const int64_t nb = ceil_div(total_q, tq), wgs = nb * num_kv_heads;
+  if (num_seqs > kOrderMax || 2 * num_kv_heads > cus) return kBlocks;
+  // a CU's share of the costs: at least with the query tokens as the only keys
+  // (the longest sequence's blocks, and one tq each for the others) ...
+  const int64_t m = std::min(ceil_div(max_q, tq), nb);
+  const int64_t least = (nb * kBlockCost + tq * (m * (m + 1) / 2 + nb - m)) * num_kv_heads / cus;
+  if (!prefers_runs(keys, least, max_q, wgs, cus)) return kBlocks;
+  // ... at most with all the keys there can be, for one causal sequence from
+  // block to block, else in every block
+  const int64_t most = (num_seqs == 1 && causal
+                            ? nb * (kBlockCost + std::max<int64_t>(keys - total_q, 0) + tq) + tq * (nb * (nb - 1) / 2)
+                            : (nb + num_seqs) * (kBlockCost + keys)) * num_kv_heads / cus;
+  return prefers_runs(std::min(keys, max_q), most, max_q, wgs, cus) ? kRuns : kEither;
 }
 
 // Words of workspace: the launch order, and the runs' part.
@@ -520,7 +530,7 @@ int64_t psk_paged_prefill_step_workspace_len(int64_t num_seqs, int64_t total_q, 
       num_q_heads % num_kv_heads || num_q_heads / num_kv_heads > kPfRows)
     return PSK_E_ARG;
   // (kRunMaxWgs: a device with fewer CUs takes the runs for no step that one with more does not)
-  const bool blocks = route(total_q, max_seqlen_q, num_seqs, num_kv_heads, kPfRows / (num_q_heads / num_kv_heads),
+  const bool blocks = route(total_q, max_seqlen_q, num_seqs, num_kv_heads, kPfRows / (num_q_heads / num_kv_heads), true,
                             max_seqlen_k, kRunMaxWgs) == kBlocks;
   return order_words(num_seqs) + (blocks ? 0 : prefill_runs_words());
 }
@@ -634,7 +644,8 @@ int psk_paged_prefill_attention(const void* q, int64_t q_tok_stride, int64_t q_h
   const int64_t cus = prefill_cus();
   const Route r = workspace_len < order_words(num_seqs) + prefill_runs_words()
                       ? kBlocks
-                      : route(total_q, max_seqlen_q, num_seqs, num_kv_heads, p.tq, block_table_width * block_size, cus);
+                      : route(total_q, max_seqlen_q, num_seqs, num_kv_heads, p.tq, a.causal != 0,
+                              block_table_width * block_size, cus);
   RunSpace space;
   int st1;
   if (r != kBlocks) {

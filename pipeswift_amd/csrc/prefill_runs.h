@@ -4,7 +4,7 @@
 // partial records that runs leave of the blocks they share.
 //
 // The host knows only how long a sequence can be (the block table's width) and
-// that the longest is no shorter than its query tokens.  Where that does not
+// that each has its query tokens at least.  Where that does not
 // settle the choice it is the device's, in two launches: prefill_runs_kernel
 // reads the lengths and either runs the step or leaves the blocks' launch
 // order, and prefill_either_kernel then merges the records or runs the blocks.
@@ -24,30 +24,41 @@ constexpr int kRunThreads = kRunWaves * 64;
 constexpr int kOrderMax = 1024;        // sequences that are ordered by length (more: batch order)
 constexpr int kRunMaxWgs = 256;        // workgroups that share a step cut into runs, at most
 
+// A query block costs kBlockCost (its queries, its first loads, its result)
+// plus the keys it reads.
+constexpr int64_t kBlockCost = 384;
+
 // Whether a step runs faster cut into equal runs than with a workgroup per
-// query block, from the longest sequence that has query tokens (`keys`), the
-// most query tokens of a sequence, the workgroups that its blocks are
-// (ceil(total_q / tq) per kv head) and the device's CUs.  Runs win where the
-// blocks are few and long: their splits, records and merge cost about 25 us,
-// which a step of short sequences does not get back.  Where the blocks fill the
-// chip several times over, or get shorter from a fresh prompt's last block to
-// its first and so fill each other's gaps, a workgroup per block is the faster:
-// on a full chip, which its power limits, that kernel takes 3-5 % less time per
-// key.  Increasing in `keys`, so a bound on the lengths decides some steps.
-// Measured, us, runs / workgroup per block, fresh prompts by query heads / kv
-// heads:
-//   tokens    250        500        1000       1400       2000       3000        4000       8000
-//   32 / 8  21.2/18.5  29.9/25.2  39.3/39.0  46.5/50.6  66.9/67.3  102.7/96.7  154/140    496/488
-//   32 / 4  22.1/18.2  29.5/25.4  37.5/39.5  49.0/51.2  69.7/68.4  103.6/95.7  155/137    498/487
-//   16 / 2  21.8/18.0  28.9/25.1  35.0/39.1  40.2/49.8  49.8/67.0   65.0/94.3  95.7/122   265/253
-//   8 / 2   21.1/18.3  28.8/24.7  32.0/38.1  33.8/49.4  40.9/65.8   48.5/93.0  61.3/120   148/231
-//   8 / 1   21.8/17.9  28.7/24.8  34.0/38.6  37.9/49.1  40.7/65.7   49.0/92.8  60.8/121   150/231
-// over a prefix (32 / 8): 64 tokens over 1000 33/42, 128 over 4096 42/126, 256
-// over 1000 35/47, 512 over 32768 264/923; six prompts of 500 beside a decode
-// of 20000 70/554; 32 / 4: seven of 600 over 20000 each 1208/2030.
-__host__ __device__ inline bool prefers_runs(int64_t keys, int64_t max_q, int64_t wgs, int64_t cus) {
-  if (keys >= 4 * max_q) return keys >= 1024 && wgs <= 4 * cus;
-  return keys >= 1536 && wgs <= cus;
+// query block, from the longest sequence that has query tokens (`keys`), a
+// CU's share of the blocks' costs, the most query tokens of a sequence, the
+// workgroups that its blocks are (ceil(total_q / tq) per kv head) and the
+// device's CUs.  A workgroup per block takes about as long as its longest
+// block, runs as long as the share; their records, merge and second start of a
+// block cost another 10-25 us, more where more blocks are shared.  So runs win
+// where the longest block stands out: any long prefix, and fresh prompts that
+// leave the chip idle.  Where the blocks fill the chip several times over, or
+// get shorter from a fresh prompt's last block to its first and so fill each
+// other's gaps, a workgroup per block is the faster.  Of 807 measured steps (1
+// to 30 sequences, 48 to 8192 new tokens over up to 45000 cached, 1 to 8 kv
+// heads) the choice takes 1.3 % more time than always taking the faster side
+// (workgroups per block alone 32 %, runs alone 11 %), and for none over 1 % more
+// than a workgroup per block.  Some of them, us, runs / workgroup per block,
+// fresh prompts by query heads / kv heads:
+//   tokens    500        1000       1400       2000       3000        4000        8000
+//   32 / 8  29.2/25.0  40.1/38.4  47.1/49.9  66.7/66.2  101.7/94.5  153/137    487/479
+//   32 / 4  28.8/25.1  38.1/39.2  48.0/50.3  69.8/66.8  102.9/93.7  155/135    493/479
+//   16 / 2  28.3/24.9  34.6/38.7  40.2/48.7  49.0/65.6   64.7/92.1  95.4/119   262/246
+//   8 / 2   28.4/24.4  31.3/37.5  33.5/48.5  38.9/65.0   47.3/90.8  60.1/117   145/226
+//   8 / 1   28.3/24.5  33.4/38.1  37.1/48.2  40.0/64.5   48.0/90.4  59.0/118   147/225
+// over a prefix (32 / 8): 64 tokens over 1000 32/42, 128 over 4096 41/126, 256
+// over 1000 35/47, 512 over 32768 260/920; six prompts of 500 beside a decode
+// of 20000 64/554; 32 / 4: seven of 600 over 20000 each 1190/2030.
+constexpr int64_t kRunsLeast = 980;  // no step of shorter sequences does
+__host__ __device__ inline bool prefers_runs(int64_t keys, int64_t share, int64_t max_q, int64_t wgs, int64_t cus) {
+  const bool prefix = keys >= 4 * max_q;  // blocks of about one length
+  if (wgs > cus) return prefix && keys >= 1024 && wgs <= 4 * cus;
+  if (keys < 1536) return keys >= kRunsLeast && share <= (keys < 1280 ? 450 : 800);
+  return prefix || keys >= 4096 || 4 * keys >= 5 * share + 1100;
 }
 
 // A value that is the same in every lane, in scalar registers.

@@ -73,7 +73,7 @@ static_assert(kPfKeys * 8 == kPfThreads, "every thread stages one 16-byte chunk 
 // least run as measured: 128, 256, 384 and 512 keys a block gave 182, 166, 161
 // and 161 us on a fresh prompt of 4000 tokens, and runs of at least 1024 or
 // 2048 took 52 and 75 us where 512 take 44 (128 tokens over 4096 keys).
-constexpr int64_t kPfCost = 384;
+constexpr int64_t kPfCost = kBlockCost;
 constexpr int kPfSnap = 3;          // a run boundary this close (in stages) to a block's end moves there
 constexpr int64_t kPfMinRun = 512;  // least cost of a run
 struct RunArgs {
@@ -165,19 +165,22 @@ struct PfStep {
   int64_t T;  // its cost
 };
 
-// Inclusive prefix over the wave.
-__device__ __forceinline__ int64_t wave_prefix(int64_t x, int lane) {
-#pragma unroll
-  for (int o = 1; o < 64; o <<= 1) {
+// Inclusive prefix and maximum over the wave's first `lanes` lanes (the maximum
+// in every lane): as many steps as they need.
+__device__ __forceinline__ int64_t wave_prefix(int64_t x, int lane, int lanes) {
+  for (int o = 1; o < lanes; o <<= 1) {
     const int64_t y = __shfl_up(x, o);
     if (lane >= o) x += y;
   }
   return x;
 }
-__device__ __forceinline__ int wave_longest(int keys) {
-#pragma unroll
-  for (int o = 1; o < 64; o <<= 1) keys = max(keys, __shfl_xor(keys, o));
+__device__ __forceinline__ int wave_longest(int keys, int lanes) {
+  for (int o = 1; o < lanes; o <<= 1) keys = max(keys, __shfl_xor(keys, o));
   return uniform(keys);
+}
+
+__device__ __forceinline__ bool pf_take(const RunArgs& p, int keys, int64_t T) {
+  return p.sure || prefers_runs(keys, T * p.a.num_kv_heads / p.cus, p.a.q_len, p.wgs, p.cus);
 }
 
 // Whether the step is cut into runs, by the threads of a workgroup (the same
@@ -192,37 +195,33 @@ __device__ __forceinline__ PfStep pf_step(const RunArgs& p, int64_t* prefix, int
   if (p.num_seqs <= 64) {
     const bool in = lane < p.num_seqs;
     const int n = in ? q_count(a, lane) : 0, len = in ? max(a.seq_lens[lane], 0) : 0;
-    if (!p.sure && !prefers_runs(wave_longest(n > 0 ? len : 0), a.q_len, p.wgs, p.cus)) {
-      if (in) put_sequence(seqs, lane, n, len);
-      return PfStep{false, 0};
+    const int keys = wave_longest(n > 0 ? len : 0, p.num_seqs);
+    PfStep found{false, 0};
+    if (p.sure || keys >= kRunsLeast) {  // else the costs do not matter
+      const PfSeq s = pf_seq(a, p.tq, n, len);
+      const int64_t x = wave_prefix(in ? s.upto(s.nb) : 0, lane, p.num_seqs);
+      if (in) prefix[lane + 1] = x;  // the same from every wave
+      const int last = p.num_seqs - 1;
+      found.T = int64_t(uint64_t(uint32_t(__builtin_amdgcn_readlane(int(x >> 32), last))) << 32 |
+                        uint32_t(__builtin_amdgcn_readlane(int(x), last)));
+      found.take = pf_take(p, keys, found.T);
     }
-    const PfSeq s = pf_seq(a, p.tq, n, len);
-    const int64_t x = wave_prefix(in ? s.upto(s.nb) : 0, lane);
-    if (in) prefix[lane + 1] = x;  // the same from every wave
-    return PfStep{true, uniform(int64_t(__shfl(x, 63)))};
+    if (!found.take && in) put_sequence(seqs, lane, n, len);
+    return found;
   }
   int keys = 0;
-  for (int b = tid; b < p.num_seqs; b += NT) {
-    const int n = q_count(a, b), len = max(a.seq_lens[b], 0);
-    put_sequence(seqs, b, n, len);
-    if (n > 0) keys = max(keys, len);
-  }
-  keys = wave_longest(keys);
-  if (lane == 0) s_wave[wave] = keys;
-  __syncthreads();
-#pragma unroll
-  for (int w = 0; w < NT / 64; ++w) keys = max(keys, int(s_wave[w]));
-  if (!p.sure && !prefers_runs(uniform(keys), a.q_len, p.wgs, p.cus)) return PfStep{false, 0};
   int64_t carry = 0;
   for (int c0 = 0; c0 < p.num_seqs; c0 += NT) {
     const int b = c0 + tid;
     int64_t own = 0;
-    if (b < p.num_seqs) {  // (the lengths that this thread read)
-      const PfSeq s = pf_seq(a, p.tq, seqs.n[b], max(seqs.key[b], 0));
+    if (b < p.num_seqs) {
+      const int n = q_count(a, b), len = max(a.seq_lens[b], 0);
+      put_sequence(seqs, b, n, len);
+      const PfSeq s = pf_seq(a, p.tq, n, len);
       own = s.upto(s.nb);
+      if (n > 0) keys = max(keys, len);
     }
-    const int64_t x = wave_prefix(own, lane);
-    __syncthreads();  // the previous values of s_wave are read
+    const int64_t x = wave_prefix(own, lane, 64);
     if (lane == 63) s_wave[wave] = x;
     __syncthreads();
     int64_t before = 0, total = 0;
@@ -233,9 +232,14 @@ __device__ __forceinline__ PfStep pf_step(const RunArgs& p, int64_t* prefix, int
     }
     if (b < p.num_seqs) prefix[b + 1] = carry + before + x;
     carry += total;
+    __syncthreads();
   }
+  keys = wave_longest(keys, 64);
+  if (lane == 0) s_wave[wave] = keys;
   __syncthreads();
-  return PfStep{true, uniform(carry)};
+#pragma unroll
+  for (int w = 0; w < NT / 64; ++w) keys = max(keys, int(s_wave[w]));
+  return PfStep{pf_take(p, uniform(keys), uniform(carry)), uniform(carry)};
 }
 
 // LDS at a byte address

@@ -9,10 +9,13 @@ KEYS, COST, SNAP, MIN_RUN, ROWS, CUS = 64, 384, 3, 512, 256, 256
 Piece = namedtuple("Piece", "b i sa sb ns")  # stages [sa, sb) of block i of sequence b, of ns
 
 
-def prefers_runs(keys, max_q, wgs, cus=CUS):
-    if keys >= 4 * max_q:
-        return keys >= 1024 and wgs <= 4 * cus
-    return keys >= 1536 and wgs <= cus
+def prefers_runs(keys, share, max_q, wgs, cus=CUS):
+    prefix = keys >= 4 * max_q
+    if wgs > cus:
+        return prefix and keys >= 1024 and wgs <= 4 * cus
+    if keys < 1536:
+        return keys >= 980 and share <= (450 if keys < 1280 else 800)
+    return prefix or keys >= 4096 or 4 * keys >= 5 * share + 1100
 
 
 def wgs(counts, Hq, Hkv, total_q=None):
@@ -20,10 +23,21 @@ def wgs(counts, Hq, Hkv, total_q=None):
     return -(-(sum(counts) if total_q is None else total_q) // tq) * Hkv
 
 
-def takes_runs(counts, lens, Hq, Hkv, total_q=None, cus=CUS):
+def cost(counts, lens, Hq, Hkv, causal=True):
+    """The step's cost per kv head."""
+    tq, total = ROWS // (Hq // Hkv), 0
+    for n, length in zip(counts, lens):
+        nb, length = -(-n // tq), max(length, 0)
+        total += nb * (COST + (max(length - n, 0) + tq if causal else length)) + (tq * nb * (nb - 1) // 2 if causal else 0)
+    return total
+
+
+def takes_runs(counts, lens, Hq, Hkv, total_q=None, causal=True, cus=CUS):
     """What the device decides (the host settles some steps before it, alike)."""
     keys = max((n for c, n in zip(counts, lens) if c > 0), default=0)
-    return len(lens) <= 1024 and 2 * Hkv <= cus and prefers_runs(keys, max(counts), wgs(counts, Hq, Hkv, total_q), cus)
+    share = cost(counts, lens, Hq, Hkv, causal) * Hkv // cus
+    return len(lens) <= 1024 and 2 * Hkv <= cus and prefers_runs(keys, share, max(counts), wgs(counts, Hq, Hkv, total_q),
+                                                                 cus)
 
 
 def runs(counts, lens, Hq, Hkv, causal, cus=CUS):

@@ -33,7 +33,7 @@ pytestmark = pytest.mark.gpu
 ])
 def test_runs(dev, Hq, Hkv, counts, prefixes, ps, causal):
     lens = [c + p for c, p in zip(counts, prefixes)]
-    assert S.takes_runs(counts, lens, Hq, Hkv, sum(counts) + 2)
+    assert S.takes_runs(counts, lens, Hq, Hkv, sum(counts) + 2, causal)
     _prefill_case(dev, 1300 + Hq + ps + len(counts), lens, counts, Hq, Hkv, ps, causal, spare_rows=2)
 
 
@@ -119,15 +119,15 @@ def test_runs_page_stride_past_32_bits(dev):
 def test_many_sequences(dev, B, long):
     """As many sequences as a wave has lanes, and more than that and than a
     workgroup has threads, empty ones among them (in keys, in queries), under a
-    table of 1100 keys: with a long sequence the step is cut into runs (two
+    table of 2000 keys: with a long sequence the step is cut into runs (two
     rounds of the scan at 700), without one the device leaves the blocks in
     launch order."""
     counts = [(i * 7) % 5 for i in range(B)]
     lens = [c + (i * 13) % 40 if i % 11 else 0 for i, c in enumerate(counts)]
-    counts[B // 2], lens[B // 2] = 6, 1100 if long else 70
+    counts[B // 2], lens[B // 2] = 6, 2000 if long else 70
     counts[0] = counts[B - 1] = 0
     assert S.takes_runs(counts, lens, 16, 2) == long
-    _prefill_case(dev, 1490 + B, lens, counts, 16, 2, 16, True, wide=1100)
+    _prefill_case(dev, 1490 + B, lens, counts, 16, 2, 16, True, wide=2000)
 
 
 def _step(dev, counts, lens, Hq, Hkv, ps=16, seed=1500):
@@ -148,7 +148,7 @@ def _step(dev, counts, lens, Hq, Hkv, ps=16, seed=1500):
 
 @pytest.mark.parametrize("counts,prefixes,Hq,Hkv,runs", [
     ([500], [0], 32, 8, False), ([250, 3], [0, 0], 32, 8, False), ([3000], [0], 32, 8, False),
-    ([500] * 8, [0] * 8, 32, 8, False), ([700, 40], [300, 500], 32, 4, False),
+    ([500] * 8, [0] * 8, 32, 8, False), ([700, 40], [250, 500], 32, 4, False),
     ([500, 1], [0, 9000], 32, 8, True), ([64], [1000], 32, 8, True), ([2000], [0], 8, 1, True),
 ])
 def test_the_lengths_choose_the_kernel(dev, counts, prefixes, Hq, Hkv, runs):

@@ -52,11 +52,11 @@ def _step_words(counts, Hq, Hkv, keys):
 @pytest.mark.parametrize("counts,Hq,Hkv,keys,records", [
     ([500], 32, 8, 500, False),          # a fresh prompt under a table of its own width
     ([500], 32, 8, 32768, True),         # the same under a wide table: the device decides
-    ([2000], 32, 8, 2000, True),
+    ([1800], 32, 8, 1800, True), ([2000], 32, 8, 2000, False), ([2000], 8, 1, 2000, True),
     ([8000], 32, 8, 1 << 20, True),      # 1000 workgroups: a long enough prefix would take the runs
     ([8001 * 5], 32, 8, 1 << 20, False),  # past four blocks a CU no length does
     ([100] * 1025, 32, 8, 4096, False),  # more sequences than the runs scan
-    ([64], 32, 8, 1023, False), ([64], 32, 8, 1024, True),
+    ([64], 32, 8, 979, False), ([64], 32, 8, 980, True),
     ([512], 512, 256, 65536, False),     # more kv heads than half the CUs
 ])
 def test_workspace_follows_the_step(counts, Hq, Hkv, keys, records):
@@ -67,28 +67,40 @@ def test_workspace_follows_the_step(counts, Hq, Hkv, keys, records):
     assert most >= 2 * B + 1
 
 
-def test_workspace_query_matches_the_rule():
-    """Against the rule itself over random steps, and refusals."""
-    r = random.Random(5)
-    for _ in range(3000):
+def test_workspace_query_allows_what_the_device_takes():
+    """Over random steps and lengths within the bound: where the device would
+    cut the step into runs, the query has asked for their records, and where
+    the query tokens are all the keys there can be it asks for no others'."""
+    r, took = random.Random(5), 0
+    for _ in range(6000):
         Hq, Hkv = r.choice(SHAPES)
-        counts = [r.randint(1, r.choice([50, 900, 9000])) for _ in range(r.randint(1, 9))]
-        keys = r.choice([0, 500, 1023, 1024, 1535, 1536, r.randint(1, 70000)])
-        want = S.prefers_runs(keys, max(counts), S.wgs(counts, Hq, Hkv))
-        assert (_step_words(counts, Hq, Hkv, keys) > 2 * len(counts) + 1) == want
+        counts = [r.randint(1, r.choice([50, 900, 9000])) for _ in range(r.choice([1, 1, 2, r.randint(1, 9)]))]
+        keys = max(counts) + r.choice([0, r.randint(0, 1500), r.randint(0, 60000)])
+        lens = [r.randint(n, keys) for n in counts]
+        if r.random() < 0.5:
+            lens[r.randrange(len(lens))] = keys
+        records = _step_words(counts, Hq, Hkv, keys) > 2 * len(counts) + 1
+        if S.takes_runs(counts, lens, Hq, Hkv, causal=r.random() < 0.7):
+            took += 1
+            assert records, (counts, lens, Hq, Hkv, keys)
+        if len(counts) == 1 and keys == counts[0]:
+            assert records == S.takes_runs(counts, counts, Hq, Hkv)
+    assert took > 500
     f = lib().psk_paged_prefill_step_workspace_len
     for bad in [(-1, 5, 5, 32, 8, 9), (1, -5, 5, 32, 8, 9), (1, 5, 0, 32, 8, 9), (1, 5, 5, 30, 8, 9),
                 (1, 5, 5, 0, 8, 9), (1, 5, 5, 32, 0, 9), (1, 5, 5, 514, 2, 9)]:
         assert f(*bad) < 0
 
 
-def test_a_bound_on_the_keys_decides_monotonically():
-    """What a longer bound refuses no shorter length takes, which is what lets
-    the host leave the records out and the longest sequence's own query tokens
-    settle a step."""
+def test_more_keys_or_less_to_share_never_refuse():
+    """What a longer bound and a smaller share refuse, no shorter length or
+    larger share takes: what lets the host settle steps."""
     r = random.Random(6)
     for _ in range(2000):
         max_q, w = r.randint(1, 20000), r.randint(1, 2000)
-        ks = sorted(r.randint(0, 90000) for _ in range(6))
-        got = [S.prefers_runs(k, max_q, w) for k in ks]
+        ks, c = sorted(r.randint(0, r.choice([2000, 90000])) for _ in range(6)), r.randint(0, 5000)
+        got = [S.prefers_runs(k, c, max_q, w) for k in ks]
         assert got == sorted(got)
+        cs = sorted(r.randint(0, 5000) for _ in range(6))
+        got = [S.prefers_runs(ks[-1], c, max_q, w) for c in cs]
+        assert got == sorted(got, reverse=True)
