@@ -420,7 +420,7 @@ def setup_prefill_attention(args, device):
     p, c = cc.prefix.double(), cc.chunk.double()
     pairs = float((c * p + c * (c + 1) / 2).sum()) * Hq  # visible (query head, key) pairs, causal
     kernel = ("decode_partial_ring_kernel + decode_combine_kernel" if fn is not attention.flash_attn_varlen_func
-              else "prefill_attention_kernel")
+              else "prefill_runs_kernel + prefill_either_kernel")
     flops = 4.0 * D * pairs
 
     def cpu_torch(budget):

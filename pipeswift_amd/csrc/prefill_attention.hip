@@ -2,7 +2,8 @@
 // attention as the decode reader of paged_attention.hip, for steps with many
 // query tokens per sequence.  The kernel here gives every query block a
 // workgroup of its own; prefill_runs.hip holds the one that cuts the step into
-// equal runs, and use_runs() chooses.
+// equal runs; prefers_runs() says which is faster, here where the bounds on the
+// lengths settle it and on the device where they do not.
 //
 // C ABI: include/pipeswift_kv.h.  Nothing here allocates or synchronizes.
 

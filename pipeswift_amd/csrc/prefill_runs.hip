@@ -45,12 +45,13 @@ namespace {
 // matrix cycles with it against 420 with 16x16.  The wave's own stream is
 // pipelined by two tiles: while the softmax of a tile runs, the scores of the
 // next one and P V of the one before are on the matrix cores (tile_step).
-// What bounds it: on a quarter of the chip a stage takes 1.5 us (start to end,
-// 8 waves; 1.7 us for the 16x16 kernel of prefill_attention.hip), on the whole
-// chip 1.9-2.0, where the clock falls to 2.15 GHz (matrix cores 50 % busy, 1.09
-// of their 2.4 GHz rate): power.  Six prefixes of 14k-45k with 4096 new tokens,
-// 32 query heads over 4 kv heads: 1400 us (1130 TFLOP/s), against 1738 with a
-// workgroup per block; 512 new tokens over 32768: 268 against 892.
+// What bounds it: power.  On a quarter of the chip a stage takes 1.5 us (start
+// to end, 8 waves; 1.7 us for the 16x16 kernel of prefill_attention.hip), on the
+// whole chip 1.9-2.0, where the clock falls to 1.8 GHz with the matrix cores 56 %
+// busy (2.2 GHz and 43 % there).  4096 new tokens over six prefixes of 14k-45k, 32
+// query heads over 4 kv heads, on five boxes: 1380-1465 us (1150-1080 TFLOP/s),
+// against 1740-1880 with a workgroup per block; 512 new tokens over 32768, 8 kv
+// heads: 257-272 against 890-924.
 constexpr int kPfWaves = kRunWaves;
 constexpr int kPfRows = kPfWaves * 32;
 static_assert(kPfRows == kBlockRows, "the blocks of both prefill kernels are the same");
@@ -69,7 +70,7 @@ static_assert(kPfKeys * 8 == kPfThreads, "every thread stages one 16-byte chunk 
 // [T j / M, T (j + 1) / M), whatever blocks it belongs to.  M x kv heads
 // workgroups, one per CU, so the chip is full and ends together however few
 // blocks a step has; a block shared by several runs leaves one partial record
-// per run (fp32 sums), merged by prefill_combine_kernel.  The cost and the
+// per run (fp32 sums), for merge_records.  The cost and the
 // least run as measured: 128, 256, 384 and 512 keys a block gave 182, 166, 161
 // and 161 us on a fresh prompt of 4000 tokens, and runs of at least 1024 or
 // 2048 took 52 and 75 us where 512 take 44 (128 tokens over 4096 keys).
