@@ -499,7 +499,8 @@ enum Route { kBlocks, kRuns, kEither };
 Route route(int64_t total_q, int64_t max_q, int64_t num_seqs, int64_t num_kv_heads, int64_t tq, bool causal,
             int64_t keys, int64_t cus) {
   const int64_t nb = ceil_div(total_q, tq), wgs = nb * num_kv_heads;
-  if (num_seqs > kOrderMax || 2 * num_kv_heads > cus) return kBlocks;
+  if (num_seqs > kOrderMax || 2 * num_kv_heads > cus || wgs > 4 * cus) return kBlocks;
+  keys = std::min<int64_t>(keys, INT32_MAX);
   // a CU's share of the costs: at least with the query tokens as the only keys
   // (the longest sequence's blocks, and one tq each for the others) ...
   const int64_t m = std::min(ceil_div(max_q, tq), nb);
@@ -527,7 +528,7 @@ int64_t psk_paged_prefill_workspace_len(int64_t num_seqs) {
 
 int64_t psk_paged_prefill_step_workspace_len(int64_t num_seqs, int64_t total_q, int64_t max_seqlen_q,
                                              int64_t num_q_heads, int64_t num_kv_heads, int64_t max_seqlen_k) {
-  if (num_seqs < 0 || total_q < 0 || max_seqlen_q <= 0 || num_kv_heads <= 0 || num_q_heads <= 0 ||
+  if (num_seqs < 0 || total_q < 0 || total_q > INT32_MAX || max_seqlen_q <= 0 || num_kv_heads <= 0 || num_q_heads <= 0 ||
       num_q_heads % num_kv_heads || num_q_heads / num_kv_heads > kPfRows)
     return PSK_E_ARG;
   // (kRunMaxWgs: a device with fewer CUs takes the runs for no step that one with more does not)

@@ -87,7 +87,8 @@ def test_workspace_query_allows_what_the_device_takes():
             assert records == S.takes_runs(counts, counts, Hq, Hkv)
     assert took > 500
     f = lib().psk_paged_prefill_step_workspace_len
-    for bad in [(-1, 5, 5, 32, 8, 9), (1, -5, 5, 32, 8, 9), (1, 5, 0, 32, 8, 9), (1, 5, 5, 30, 8, 9),
+    assert f(1, 500, 500, 32, 8, (1 << 63) - 1) == lib().psk_paged_prefill_workspace_len(1)  # lengths not known
+    for bad in [(-1, 5, 5, 32, 8, 9), (1, -5, 5, 32, 8, 9), (1, 1 << 31, 5, 32, 8, 9), (1, 5, 0, 32, 8, 9), (1, 5, 5, 30, 8, 9),
                 (1, 5, 5, 0, 8, 9), (1, 5, 5, 32, 0, 9), (1, 5, 5, 514, 2, 9)]:
         assert f(*bad) < 0
 
