@@ -197,11 +197,11 @@ struct MergeLds {
 // block and kv head, so that the wave's 4 KiB of a record are in flight at
 // once; the tasks of the blocks there are go round the launch's workgroups,
 // then their waves, so that a few use every CU's share of the bandwidth.
-// R records' columns are in flight at a time.  Bound by the latency of what
-// other XCDs have just written, 1-2 us a round of loads, so the rounds count:
-// with the tasks on the first workgroups, four records a round and each round's
-// maxima before it, 7 sequences of 4-11k cached tokens (one kv head a rank, 14
-// records a block) took 52.1 us for 39.3, a prompt of 2000 on 8 kv heads 66.7 for 65.3.
+// R records' columns are in flight at a time.  Bound by the latency of the loads, so the
+// rounds of them count: 7 appends of 11-65 tokens over 4-11k cached, 8 query heads on
+// 2 kv heads, the whole call with this merge in the launch the device chooses for:
+// 54.7 us with the tasks on the first workgroups, 50.6-52.2 spread over all of them
+// (R = 4 and 8), 42.1 (R = 4) and 39.3 (R = 8) with the maxima 16 a round as well.
 template <int OUT_DT, int R>
 __device__ __forceinline__ void merge_records(const DecodeArgs& a, int tq, const RunSpace& s, MergeLds& lds) {
   const int tid = int(threadIdx.x), lane = tid & 63, wave = uniform(tid >> 6);
